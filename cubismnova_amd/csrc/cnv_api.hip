@@ -68,6 +68,9 @@ int ensure_bc_table(cnv_grid_s *g, int comp)
             entries.push_back({bc.kind, bc.dir, bc.side, 0, bc.value});
             any = true;
         }
+        const int sb[3] = {-1, -1, -1}, se[3] = {2, 2, 2};
+        resolve_faces(entries.data() + heads[(size_t)b].offset, (int)lst.size(), sb, se, heads[(size_t)b].kind,
+                      heads[(size_t)b].val);
     }
     if (t.heads || t.entries) {
         // the table is rewritten (BC lists changed): kernels still queued on

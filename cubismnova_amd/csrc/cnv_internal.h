@@ -37,10 +37,14 @@ struct DevBC {
     double value;
 };
 
-// Per-block header into the flattened BC entry array.
+// Per-block header into the flattened BC entry array, with the block's six
+// faces resolved (FaceKind and the Dirichlet constant or Symmetry sign; the
+// same for every stencil that reads ghosts on both sides of each dimension).
 struct DevBCHead {
     int offset;
     int count;
+    int kind[6];
+    double val[6];
 };
 
 // Face of a block as the non-tensorial operator kernels see it after the

@@ -1,0 +1,59 @@
+"""GPU parity of the column kernels (block shapes outside 16, 32 and 64 cells
+per x/y edge) against the oracle, bit for bit, at the shapes where a lane
+numbering can go wrong: rows of one vector, rows that no vector divides,
+planes smaller and larger than a workgroup, one-cell and one-block directions,
+chunks with a remainder, components with different BC lists."""
+import numpy as np
+import pytest
+
+import cubismnova_amd as cnv
+import oracle
+from tests.helpers import assert_same, cells_of, face_bc_lists, random_slab
+
+pytestmark = pytest.mark.gpu
+
+KIND = {0: cnv.Base, 1: cnv.Absorbing, 2: cnv.Dirichlet, 3: cnv.Symmetry}
+MIXED = [(2, 0, 0, 0.75), (3, 0, 1, -1.0), (1, 1, 0, 0.0), (3, 1, 1, 1.0), (2, 2, 0, -0.5), (1, 2, 1, 0.0)]
+PARTLY = [(1, 2, 0, 0.0), (3, 2, 1, -0.5)]
+SHAPES = [((2, 2, 2), (8, 8, 8)), ((3, 2, 2), (4, 12, 9)), ((1, 1, 1), (5, 7, 3)), ((2, 3, 1), (6, 5, 33)),
+          ((1, 2, 2), (24, 24, 24)), ((2, 1, 2), (40, 13, 6)), ((1, 1, 3), (1, 1, 1)), ((2, 1, 1), (65, 64, 5)),
+          ((7, 5, 3), (8, 8, 8))]
+
+
+def build(nb, n, dtype, seed, lists):
+    """Grid of one component per BC list, its slabs and per-component lists."""
+    g = cnv.Cartesian(nb, n, dtype=dtype, ncomp=len(lists))
+    slabs, bcs = [], []
+    for c, faces in enumerate(lists):
+        slab = random_slab(seed + c, nb, n, dtype, g.block_stride)
+        g.upload(c, slab)
+        bcl = face_bc_lists(nb, faces)
+        for b, lst in bcl.items():
+            bi = (b % nb[0], (b // nb[0]) % nb[1], b // (nb[0] * nb[1]))
+            g.setBC(bi, [KIND[k](d, s, v) if k in (2, 3) else KIND[k](d, s) for k, d, s, v in lst], comp=c)
+        slabs.append(slab)
+        bcs.append(bcl)
+    return g, slabs, bcs
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+@pytest.mark.parametrize("lists", [[[]], [MIXED, [], PARTLY]], ids=["periodic", "walls"])
+def test_diffusion_columns(gpu, dtype, shape, lists):
+    nb, n = shape
+    g, slabs, bcs = build(nb, n, dtype, 7, lists)
+    out = cnv.Cartesian(nb, n, dtype=dtype, ncomp=len(lists))
+    lap = cnv.Cartesian(nb, n, dtype=dtype, ncomp=len(lists))
+    h = [1.0 / (nb[d] * n[d]) for d in range(3)]
+    dt = 0.1 * min(h) ** 2
+    s = cnv.DeviceBuffer(8)
+    cnv.diffusion_step(g, out, dt, lap=lap, sumsq=s)
+    tot = 0.0
+    for c, slab in enumerate(slabs):
+        f = oracle.Field(slab, nb, n, g.block_stride, bcs=bcs[c])
+        un, sref, lref = oracle.diffusion_step(f, h, dt, want_lap=True)
+        tot += sref
+        assert_same(cells_of(out.download(c), nb, n, g.block_stride), cells_of(un, nb, n, g.block_stride), "euler")
+        assert_same(cells_of(lap.download(c), nb, n, g.block_stride), cells_of(lref, nb, n, g.block_stride), "lap")
+    # the FP64 sum in another order: 1e-13 of it, as everywhere
+    assert abs(s.download(np.float64, 1)[0] - tot) <= 1e-13 * tot

@@ -258,10 +258,12 @@ struct S7Tune {
 static std::mutex g_tune_mtx;
 static std::map<std::tuple<int, int>, S7Tune> g_tune; // (dtype, edge) -> choice
 
-S7Tune s7_default_tune(int dtype, int edge)
+S7Tune s7_default_tune(int dtype, int edge, bool *pinned = nullptr)
 {
     std::lock_guard<std::mutex> lk(g_tune_mtx);
     auto it = g_tune.find({dtype, edge});
+    if (pinned)
+        *pinned = it != g_tune.end();
     if (it != g_tune.end())
         return it->second;
     if (edge >= 64)
@@ -372,6 +374,21 @@ static int run_cols(S7Args &a, int ncomp, hipStream_t st, bool finalize, int *np
     return CNV_OK;
 }
 
+// Grids of 16, 32 or 64 cells per x/y edge run as columns up to 40 MB of
+// input unless a tile is pinned: the marching tiles step through 8 or 16
+// planes one after another, and on a small grid too few of them run at once
+// to cover that chain's latency.  Per Euler step with its norm (marching
+// tile / columns): 64^3 FP64 in 16^3 blocks 10.9 / 6.1 us, 128^3 FP64 in 32^3
+// blocks 15.1 / 11.7, 64^3 FP32 in one 64^3 block 19.7 / 5.3, 192^3 FP32 (28
+// MB) 17.6 / 16.9 in 32^3 and 23.7 / 17.3 in 64^3 blocks; 192^3 FP64 (57 MB)
+// 28.6 / 26.1 in 16^3 but 24.2 / 25.3 in 32^3 blocks, and 256^3 FP64 49.9 /
+// 59.2.
+static bool cols_for_small(const Geom &G, int ncomp, size_t elem)
+{
+    const long long cells = (long long)G.nb[0] * G.nb[1] * G.nb[2] * ncomp * G.n[0] * G.n[1] * G.n[2];
+    return cells * (long long)elem < 40ll * 1000 * 1000;
+}
+
 // cap: partials the buffer at a.partials holds (0: sized by the caller for
 // the largest launch)
 template <typename T, int MODE, bool SUMSQ>
@@ -382,7 +399,10 @@ static int run_t(S7Args &a, int ncomp, hipStream_t st, int force_generic, const 
     const long long nbt = (long long)a.G.nb[0] * a.G.nb[1] * a.G.nb[2];
     const bool cubic_xy = n[0] == n[1];
     if (!force_generic && cubic_xy && (n[0] == 16 || n[0] == 32 || n[0] == 64)) {
-        S7Tune tu = over ? *over : s7_default_tune(sizeof(T) == 8 ? CNV_F64 : CNV_F32, n[0]);
+        bool pinned = false;
+        S7Tune tu = over ? *over : s7_default_tune(sizeof(T) == 8 ? CNV_F64 : CNV_F32, n[0], &pinned);
+        if (!over && !pinned && cols_for_small(a.G, ncomp, sizeof(T)))
+            return run_cols<T, MODE, SUMSQ>(a, ncomp, st, finalize, nparts, cap);
         a.zchunk = tu.zchunk < n[2] ? tu.zchunk : n[2];
         a.nzc = (n[2] + a.zchunk - 1) / a.zchunk;
         a.tiles_per_comp = (int)(nbt * a.nzc);

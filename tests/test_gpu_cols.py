@@ -1,5 +1,5 @@
 """GPU parity of the column kernels (block shapes outside 16, 32 and 64 cells
-per x/y edge) against the oracle, bit for bit, at the shapes where a lane
+per x/y edge, and small grids of those) against the oracle, bit for bit, at the shapes where a lane
 numbering can go wrong: rows of one vector, rows that no vector divides,
 planes smaller and larger than a workgroup, one-cell and one-block directions,
 chunks with a remainder, components with different BC lists."""
@@ -17,7 +17,7 @@ MIXED = [(2, 0, 0, 0.75), (3, 0, 1, -1.0), (1, 1, 0, 0.0), (3, 1, 1, 1.0), (2, 2
 PARTLY = [(1, 2, 0, 0.0), (3, 2, 1, -0.5)]
 SHAPES = [((2, 2, 2), (8, 8, 8)), ((3, 2, 2), (4, 12, 9)), ((1, 1, 1), (5, 7, 3)), ((2, 3, 1), (6, 5, 33)),
           ((1, 2, 2), (24, 24, 24)), ((2, 1, 2), (40, 13, 6)), ((1, 1, 3), (1, 1, 1)), ((2, 1, 1), (65, 64, 5)),
-          ((7, 5, 3), (8, 8, 8))]
+          ((7, 5, 3), (8, 8, 8)), ((2, 1, 2), (16, 16, 16)), ((1, 2, 1), (32, 32, 32)), ((1, 1, 2), (64, 64, 6))]
 
 
 def build(nb, n, dtype, seed, lists):
@@ -57,3 +57,17 @@ def test_diffusion_columns(gpu, dtype, shape, lists):
         assert_same(cells_of(lap.download(c), nb, n, g.block_stride), cells_of(lref, nb, n, g.block_stride), "lap")
     # the FP64 sum in another order: 1e-13 of it, as everywhere
     assert abs(s.download(np.float64, 1)[0] - tot) <= 1e-13 * tot
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("edge,tile", [(16, (128, 8)), (32, (256, 8)), (64, (512, 16))])
+def test_pinned_tile_on_a_small_grid(gpu, dtype, edge, tile):
+    """A pinned tile keeps the marching kernel where the columns would run."""
+    nb, n = (2, 1, 2), (edge, edge, edge)
+    g, slabs, bcs = build(nb, n, dtype, 11, [MIXED])
+    out = cnv.Cartesian(nb, n, dtype=dtype)
+    cnv.set_tune_stencil7(dtype, edge, *tile)
+    cnv.diffusion_step(g, out, 1e-6)
+    h = [1.0 / (nb[d] * n[d]) for d in range(3)]
+    un, _ = oracle.diffusion_step(oracle.Field(slabs[0], nb, n, bcs=bcs[0]), h, 1e-6)
+    assert_same(out.download(0), un)

@@ -219,6 +219,7 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
 // two Euler steps per launch on periodic grids (cnv_stencil7x2.hip)
 bool x2_applicable(cnv_grid_s *u);
 long long x2_tiles(const cnv_grid_s *u, int zchunk);
+void x2_tile(cnv_grid_s *u, int *wg, int *zchunk);
 int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *part1, double *part2,
                         const double *const prev_p[2], const int prev_n[2], double *const prev_out[2], int wg,
                         int zchunk, int *nparts, hipStream_t st);

@@ -655,7 +655,7 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
     const size_t cap = u->partials_cap;
     int nfused = 0, xwg = 0, xz = 0;
     if (nsteps >= 4 && !force_generic() && x2_applicable(u) && x2_applicable(tmp)) {
-        x2_get_tune(u->desc.dtype, u->desc.block_cells[0], &xwg, &xz);
+        x2_tile(u, &xwg, &xz);
         if (2 * x2_tiles(u, xz) <= (long long)cap)
             nfused = 2 * (nsteps / 4);
     }

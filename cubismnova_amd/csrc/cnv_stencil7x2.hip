@@ -419,14 +419,26 @@ X2Tune x2_default(int dtype, int edge)
     return dtype == CNV_F64 ? X2Tune{128, 16} : X2Tune{64, 16};
 }
 
-X2Tune x2_tune(int dtype, int edge)
+X2Tune x2_tune(int dtype, int edge, bool *pinned = nullptr)
 {
     std::lock_guard<std::mutex> lk(g_x2_mtx);
     auto it = g_x2_tune.find({dtype, edge});
+    if (pinned)
+        *pinned = it != g_x2_tune.end();
     return it == g_x2_tune.end() ? x2_default(dtype, edge) : it->second;
 }
 
-// z-chunks compiled: 8, 16 and 32 planes (up to the block edge)
+// Tiles a launch needs to fill the GPU with the built-in workgroup size
+// (fewer where a tile has more waves or more LDS).
+int x2_enough(int dtype, int edge)
+{
+    if (edge == 32)
+        return dtype == CNV_F64 ? 400 : 600;
+    return dtype == CNV_F64 ? 800 : 1500;
+}
+
+// z-chunks that can be pinned: 8, 16 and 32 planes (up to the block edge);
+// chunks of 2 and 4 planes are compiled for small grids
 inline bool x2_zchunk_ok(int zc) { return zc == 8 || zc == 16 || zc == 32; }
 
 template <typename T, int N, int WG>
@@ -437,6 +449,10 @@ bool x2_launch1(const X2Args &a, int zc, int ntiles, hipStream_t st)
             hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 16>), dim3(ntiles), dim3(WG), 0, st, a);
         else if (zc == 8)
             hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 8>), dim3(ntiles), dim3(WG), 0, st, a);
+        else if (zc == 4)
+            hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 4>), dim3(ntiles), dim3(WG), 0, st, a);
+        else if (zc == 2)
+            hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 2>), dim3(ntiles), dim3(WG), 0, st, a);
         else if constexpr (N == 32) {
             if (zc != 32)
                 return false;
@@ -535,7 +551,7 @@ int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *pa
     a.u = static_cast<const char *>(u->data);
     a.out = static_cast<char *>(out->data);
     a.G = geom_of(u);
-    if (!x2_zchunk_ok(zchunk))
+    if (!x2_zchunk_ok(zchunk) && zchunk != 2 && zchunk != 4)
         return fail(CNV_ERR_UNSUPPORTED, "two-step kernel: zchunk must be 8, 16 or 32");
     if (zchunk > edge)
         return fail(CNV_ERR_UNSUPPORTED, "two-step kernel: zchunk larger than the block edge");
@@ -583,6 +599,26 @@ int x2_get_tune(int dtype, int edge, int *wg, int *zchunk)
     if (zchunk)
         *zchunk = t.zchunk;
     return CNV_OK;
+}
+
+// The tile of a run on this grid: the pinned one, else the built-in workgroup
+// size with the deepest z chunk that gives enough tiles, down to two planes.  A chunk of zc planes
+// marches zc + 2 planes one after another, each about 0.9 us (one barrier,
+// one exposed load), so on a small grid the chain is the launch: 64^3 FP64 in
+// 16^3 blocks 8.1 / 5.1 / 4.1 / 3.6 us per step with 16 / 8 / 4 / 2 planes,
+// 128^3 FP32 in 32^3 blocks 9.4 / 6.0 / 5.0 / 5.0.  A shallow chunk reads and
+// evaluates more halo planes, which costs once the GPU is full: 256^3 FP32
+// 14.6 / 17.7 / 21.3 / 25.7, 192^3 FP64 13.1 / 15.5 / 18.0 / 21.6 in 32^3 blocks.
+void x2_tile(cnv_grid_s *u, int *wg, int *zchunk)
+{
+    const int dtype = u->desc.dtype, edge = u->desc.block_cells[0];
+    bool pinned = false;
+    X2Tune t = x2_tune(dtype, edge, &pinned);
+    if (!pinned)
+        while (t.zchunk > 2 && x2_tiles(u, t.zchunk) < x2_enough(dtype, edge))
+            t.zchunk /= 2;
+    *wg = t.wg;
+    *zchunk = t.zchunk;
 }
 
 // Times every valid (workgroup size, z-planes per tile) pair of the two-step

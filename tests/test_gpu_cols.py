@@ -71,3 +71,27 @@ def test_pinned_tile_on_a_small_grid(gpu, dtype, edge, tile):
     h = [1.0 / (nb[d] * n[d]) for d in range(3)]
     un, _ = oracle.diffusion_step(oracle.Field(slabs[0], nb, n, bcs=bcs[0]), h, 1e-6)
     assert_same(out.download(0), un)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("nb,edge", [((1, 1, 1), 16), ((3, 2, 1), 16), ((9, 8, 7), 16), ((2, 1, 3), 32),
+                                     ((6, 5, 3), 32)])
+def test_run_depth_by_grid_size(gpu, dtype, nb, edge):
+    """diffusion_run picks the two-step kernel's z chunk (2, 4 or 8 planes
+    here) from the grid's tile count: fields equal to single steps bit for
+    bit, norms to 1e-13 (another summation order)."""
+    n = (edge,) * 3
+    slab = random_slab(17, nb, n, dtype)
+    u, t, v, w = (cnv.Cartesian(nb, n, dtype=dtype) for _ in range(4))
+    u.upload(0, slab)
+    v.upload(0, slab)
+    dt = 0.1 / (edge * max(nb)) ** 2
+    norms, want = cnv.DeviceBuffer(8 * 6), cnv.DeviceBuffer(8 * 6)
+    res = cnv.diffusion_run(u, t, 6, dt, norms)
+    a, b = v, w
+    for k in range(6):
+        cnv.diffusion_step(a, b, dt, sumsq=want.at(8 * k))
+        a, b = b, a
+    assert_same(res.download(0), a.download(0))
+    gn, wn = norms.download(np.float64, 6), want.download(np.float64, 6)
+    assert np.max(np.abs(gn - wn) / wn) <= 1e-13

@@ -735,11 +735,43 @@ static J2Tune j2_default(int dtype, int edge)
 static std::mutex g_j2_mtx;
 static std::map<std::pair<int, int>, J2Tune> g_j2_tune;
 
-static J2Tune j2_tune(int dtype, int edge)
+// pinned: set to something else than the built-in tile
+static J2Tune j2_tune(int dtype, int edge, bool *pinned = nullptr)
 {
     std::lock_guard<std::mutex> lk(g_j2_mtx);
     auto it = g_j2_tune.find({dtype, edge});
-    return it == g_j2_tune.end() ? j2_default(dtype, edge) : it->second;
+    const J2Tune d = j2_default(dtype, edge), t = it == g_j2_tune.end() ? d : it->second;
+    if (pinned)
+        *pinned = t.wg != d.wg || t.zchunk != d.zchunk || t.split != d.split;
+    return t;
+}
+
+// The tile of a launch on `nbt` blocks of nz planes: the pinned one, else the
+// built-in one with the deepest z chunk (down to two planes) that gives enough
+// tiles to fill the GPU.  A chunk of z planes marches z + 2 planes one after
+// another, so on a small grid the chain is the launch.  Us per launch of two
+// sweeps, built-in depth / this rule: 64^3 FP32 in 32^3 blocks 55.4 / 8.4,
+// 128^3 FP32 in 64^3 blocks 217 / 12.8, 256^3 FP32 in 64^3 blocks 227 / 50,
+// 192^3 FP64 in 32^3 blocks 76 / 50, 128^3 FP64 in 16^3 blocks 30.1 / 20.7.
+// Enough is two 64-edge tiles per CU (LDS lets no more run at once) and as
+// many waves of the smaller ones: half that many tiles, or twice, is slower
+// (256^3 FP32 in 32^3 blocks, 32 / 16 / 8 planes: 74.6 / 55.4 / 63.9).
+static J2Tune j2_tile(int dtype, int edge, long long nbt, int nz)
+{
+    bool pinned = false;
+    J2Tune t = j2_tune(dtype, edge, &pinned);
+    if (pinned)
+        return t;
+    long long enough = edge >= 64 || (edge == 32 && dtype == CNV_F64) ? 400 : edge == 32 ? 600 : 1500;
+    if (edge == 16 && dtype == CNV_F64)
+        t.wg = 64; // one wave per tile: 256^3 118 against 140 us with two
+    auto tiles = [&](int z) { return nbt * ((nz + z - 1) / z) * t.split; };
+    t.zchunk = std::min(t.zchunk, nz);
+    while (t.zchunk > 2 && tiles(t.zchunk) < enough)
+        t.zchunk = (t.zchunk + 1) / 2;
+    if (edge >= 64 && tiles(t.zchunk) < enough)
+        t.wg = 512; // too few tiles at any depth: more waves in each (128^3 FP32 15.7 -> 12.8 us)
+    return t;
 }
 
 int jacobi2_set_tune(int dtype, int edge, int wg, int zchunk, int split)
@@ -885,7 +917,8 @@ int launch_jacobi2(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out
     a.ihx2 = 1. / (u->h[0] * u->h[0]);
     a.ihy2 = 1. / (u->h[1] * u->h[1]);
     a.omega = omega;
-    const J2Tune tu = tile ? J2Tune{tile[0], tile[1], tile[2]} : j2_tune(u->desc.dtype, n[0]);
+    const J2Tune tu = tile ? J2Tune{tile[0], tile[1], tile[2]}
+                            : j2_tile(u->desc.dtype, n[0], u->nblocks_total, n[2]);
     a.zchunk = std::min(std::min(tu.zchunk, n[2]), kJ2ZMax);
     a.nzc = (n[2] + a.zchunk - 1) / a.zchunk;
     const long long ntiles = u->nblocks_total * a.nzc * tu.split;

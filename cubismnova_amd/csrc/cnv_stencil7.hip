@@ -258,21 +258,22 @@ struct S7Tune {
 static std::mutex g_tune_mtx;
 static std::map<std::tuple<int, int>, S7Tune> g_tune; // (dtype, edge) -> choice
 
+// The tile in use; pinned: set to something else than the built-in one.
 S7Tune s7_default_tune(int dtype, int edge, bool *pinned = nullptr)
 {
+    S7Tune d{64, 8};
+    if (edge >= 64)
+        d = {512, 16};
+    else if (edge >= 32)
+        d = {256, 8};
+    else if (dtype == CNV_F64)
+        d = {128, 8};
     std::lock_guard<std::mutex> lk(g_tune_mtx);
     auto it = g_tune.find({dtype, edge});
+    const S7Tune t = it == g_tune.end() ? d : it->second;
     if (pinned)
-        *pinned = it != g_tune.end();
-    if (it != g_tune.end())
-        return it->second;
-    if (edge >= 64)
-        return {512, 16};
-    if (edge >= 32)
-        return {256, 8};
-    if (dtype == CNV_F64)
-        return {128, 8};
-    return {64, 8};
+        *pinned = t.wg != d.wg || t.zchunk != d.zchunk;
+    return t;
 }
 
 void s7_set_tune(int dtype, int edge, int wg, int zchunk)

@@ -419,13 +419,15 @@ X2Tune x2_default(int dtype, int edge)
     return dtype == CNV_F64 ? X2Tune{128, 16} : X2Tune{64, 16};
 }
 
+// pinned: set to something else than the built-in tile
 X2Tune x2_tune(int dtype, int edge, bool *pinned = nullptr)
 {
     std::lock_guard<std::mutex> lk(g_x2_mtx);
     auto it = g_x2_tune.find({dtype, edge});
+    const X2Tune d = x2_default(dtype, edge), t = it == g_x2_tune.end() ? d : it->second;
     if (pinned)
-        *pinned = it != g_x2_tune.end();
-    return it == g_x2_tune.end() ? x2_default(dtype, edge) : it->second;
+        *pinned = t.wg != d.wg || t.zchunk != d.zchunk;
+    return t;
 }
 
 // Tiles a launch needs to fill the GPU with the built-in workgroup size

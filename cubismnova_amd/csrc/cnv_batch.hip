@@ -41,7 +41,6 @@ struct BGrid {
     int op, g, ncomp, pad;
     int has_bc[kBMaxComp];
     const DevBCHead *heads[kBMaxComp];
-    const DevBC *entries[kBMaxComp];
     float ih2[3];
     float nudt;
 };
@@ -97,8 +96,7 @@ __device__ __attribute__((always_inline)) inline void gen_item(const BGrid *__re
     const float *cbase = Gd.in + (long long)c * Gd.G.cstride;
     const float *ub = cbase + (long long)I.blk * Gd.G.bstride;
     FaceL<float> F[6];
-    const int sb[3] = {-Gd.g, -Gd.g, -Gd.g}, se[3] = {Gd.g + 1, Gd.g + 1, Gd.g + 1};
-    make_faces<float>(Gd.G, Gd.heads[c], Gd.entries[c], Gd.has_bc[c], I.blk, cbase, sb, se, F);
+    make_faces<float>(Gd.G, Gd.heads[c], Gd.has_bc[c], I.blk, cbase, F);
     const long long sx = nx, sxy = (long long)nx * ny;
     // stage the tile and its face halo, U cells per thread and pass: their
     // loads are all issued before the first LDS store, so they are in
@@ -192,7 +190,7 @@ __device__ __attribute__((always_inline)) inline void s7_item(const BGrid *__res
     const float *ub = cbase + (long long)I.blk * Gd.G.bstride;
     float *ob = Gd.out + (long long)I.blk * Gd.G.bstride;
     FaceSrc<float> F[6];
-    block_faces<float>(Gd.G, Gd.heads[c], Gd.entries[c], Gd.has_bc[c], I.blk, cbase, F);
+    block_faces<float>(Gd.G, Gd.heads[c], Gd.has_bc[c], I.blk, cbase, F);
     (void)s7_march<float, NX, NX, WG, 1, false, SUB>(ub, ob + (long long)c * Gd.ocstride, nullptr, F, NX, I.z0,
                                                       I.z0 + I.nz, Gd.ih2[0], Gd.ih2[1], Gd.ih2[2], Gd.nudt, lds);
 }
@@ -207,8 +205,7 @@ __device__ __attribute__((always_inline)) inline void w5_item(const BGrid *__res
     const float *ub = cbase + (long long)I.blk * Gd.G.bstride;
     float *ob = Gd.out + (long long)I.blk * Gd.G.bstride;
     FaceL<float> F[6];
-    const int sb[3] = {-Gd.g, -Gd.g, -Gd.g}, se[3] = {Gd.g + 1, Gd.g + 1, Gd.g + 1};
-    make_faces<float>(Gd.G, Gd.heads[c], Gd.entries[c], Gd.has_bc[c], I.blk, cbase, sb, se, F);
+    make_faces<float>(Gd.G, Gd.heads[c], Gd.has_bc[c], I.blk, cbase, F);
     w5_march<float, NX, NX, WG, SUB>(ub, ob + (long long)(6 * c) * Gd.ocstride, Gd.ocstride, F, NX, I.z0,
                                      I.z0 + I.nz, lds);
 }
@@ -565,9 +562,8 @@ static int build_grids(cnv_batch_s *b)
             if (rc != CNV_OK)
                 return rc;
             const BCTable &t = g->tables[c];
-            d.has_bc[c] = (t.any && t.heads && t.entries) ? 1 : 0;
+            d.has_bc[c] = (t.any && t.heads) ? 1 : 0;
             d.heads[c] = t.heads;
-            d.entries[c] = t.entries;
             // every face the operator reads must be written by the lab rules
             const int sb[3] = {-it.ghost, -it.ghost, -it.ghost}, se[3] = {it.ghost + 1, it.ghost + 1, it.ghost + 1};
             for (const auto &l : g->bcs[c]) {

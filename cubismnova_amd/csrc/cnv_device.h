@@ -164,24 +164,18 @@ __device__ inline T face_val(const FaceSrc<T> &f, long long i)
 // Resolve the six one-layer faces of block `blk` (ghost layer 1 of the lab,
 // the only one the 7-point operators read; the same for any ghost width).
 template <typename T>
-__device__ inline void block_faces(const Geom &G, const DevBCHead *heads, const DevBC *entries, int has_bc,
-                                   long long blk, const T *cbase, FaceSrc<T> F[6])
+__device__ inline void block_faces(const Geom &G, const DevBCHead *heads, int has_bc, long long blk, const T *cbase,
+                                   FaceSrc<T> F[6])
 {
     const int *nb = G.nb, *n = G.n;
     const int bidx[3] = {(int)(blk % nb[0]), (int)((blk / nb[0]) % nb[1]),
                          (int)(blk / ((long long)nb[0] * nb[1]))};
     int kind[6];
     double val[6];
-    const int sb[3] = {-1, -1, -1}, se[3] = {2, 2, 2};
-    if (has_bc) {
-        const DevBCHead h = heads[blk];
-        resolve_faces(entries + h.offset, h.count, sb, se, kind, val);
-    } else {
 #pragma unroll
-        for (int f = 0; f < 6; ++f) {
-            kind[f] = FACE_NBR;
-            val[f] = 0.0;
-        }
+    for (int f = 0; f < 6; ++f) {
+        kind[f] = has_bc ? heads[blk].kind[f] : FACE_NBR;
+        val[f] = has_bc ? heads[blk].val[f] : 0.0;
     }
     const long long nx = n[0], nxy = (long long)n[0] * n[1];
     const T *self = cbase + blk * G.bstride;
@@ -269,26 +263,21 @@ __device__ inline T face_layer(const FaceL<T> &f, int l, long long dstride, long
     return f.mode == 1 ? f.s * v : v;
 }
 
-// Six faces of block `blk` for a non-tensorial stencil (sb, se) from the
-// block's BC list (heads/entries may be null when no block carries a BC).
+// Six faces of block `blk` for a non-tensorial stencil from the block's
+// resolved faces (heads may be null when no block carries a BC).
 template <typename T>
-__device__ inline void make_faces(const Geom &G, const DevBCHead *heads, const DevBC *entries, int has_bc,
-                                  long long blk, const T *cbase, const int sb[3], const int se[3], FaceL<T> F[6])
+__device__ inline void make_faces(const Geom &G, const DevBCHead *heads, int has_bc, long long blk, const T *cbase,
+                                  FaceL<T> F[6])
 {
     const int *nb = G.nb, *n = G.n;
     const int bidx[3] = {(int)(blk % nb[0]), (int)((blk / nb[0]) % nb[1]),
                          (int)(blk / ((long long)nb[0] * nb[1]))};
     int kind[6];
     double val[6];
-    if (has_bc) {
-        const DevBCHead h = heads[blk];
-        resolve_faces(entries + h.offset, h.count, sb, se, kind, val);
-    } else {
 #pragma unroll
-        for (int f = 0; f < 6; ++f) {
-            kind[f] = FACE_NBR;
-            val[f] = 0.0;
-        }
+    for (int f = 0; f < 6; ++f) {
+        kind[f] = has_bc ? heads[blk].kind[f] : FACE_NBR;
+        val[f] = has_bc ? heads[blk].val[f] : 0.0;
     }
     const T *self = cbase + blk * G.bstride;
 #pragma unroll

@@ -33,7 +33,6 @@ struct JArgs {
     int nzc, zchunk;
     int has_bc;
     const DevBCHead *heads;
-    const DevBC *entries;
     const double *czm, *czp; // per global z cell
     double ihx2, ihy2, omega;
     double *partials;
@@ -73,8 +72,7 @@ __global__ __launch_bounds__(WG) void k_jacobi(const JArgs a)
     TO *ob = reinterpret_cast<TO *>(a.out) + (long long)a.co * a.cs_o + blk * a.bs_o;
 
     FaceL<T> F[6];
-    const int sb[3] = {-1, -1, -1}, se[3] = {2, 2, 2};
-    make_faces<T>(a.G, a.heads, a.entries, a.has_bc, blk, cbase, sb, se, F);
+    make_faces<T>(a.G, a.heads, a.has_bc, blk, cbase, F);
 
     const int tx = tid % TX, ty = tid / TX;
     const int x0 = tx * VEC;
@@ -499,9 +497,8 @@ int launch_jacobi(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out,
                     return fail(CNV_ERR_UNSUPPORTED, "BC list leaves ghost cells unwritten");
         }
         const BCTable &t = u->tables[cu];
-        a.has_bc = (t.any && t.heads && t.entries) ? 1 : 0;
+        a.has_bc = (t.any && t.heads) ? 1 : 0;
         a.heads = t.heads;
-        a.entries = t.entries;
     }
     a.u = static_cast<const char *>(u->data);
     a.f = static_cast<const char *>(f->data);

@@ -38,7 +38,6 @@ struct S7Args {
     int tiles_per_comp;
     int has_bc[kMaxComp];
     const DevBCHead *heads[kMaxComp];
-    const DevBC *entries[kMaxComp];
     double ih2[3];
     double nudt;
     double *partials;
@@ -80,7 +79,7 @@ __global__ __launch_bounds__(WG) void k_stencil7(const S7Args a)
                       : nullptr;
 
     FaceSrc<T> F[6];
-    block_faces<T>(a.G, a.heads[comp], a.entries[comp], a.has_bc[comp], blk, cbase, F);
+    block_faces<T>(a.G, a.heads[comp], a.has_bc[comp], blk, cbase, F);
     double acc = s7_march<T, NX, NY, WG, MODE, SUMSQ>(ub, ob, lb, F, NZ, z0, z1, (T)a.ih2[0], (T)a.ih2[1],
                                                       (T)a.ih2[2], (T)a.nudt, lds);
 
@@ -499,7 +498,6 @@ static int launch_stencil7_t(cnv_grid_s *u, cnv_grid_s *out, cnv_grid_s *lap, in
     for (int c = 0; c < ncomp; ++c) {
         a.has_bc[c] = 0;
         a.heads[c] = nullptr;
-        a.entries[c] = nullptr;
     }
     if (!u->tables.empty()) { // a grid without tables is periodic on every face
         std::lock_guard<std::mutex> lk(u->mtx);
@@ -511,15 +509,13 @@ static int launch_stencil7_t(cnv_grid_s *u, cnv_grid_s *out, cnv_grid_s *lap, in
             if (rc != CNV_OK)
                 return rc;
             const BCTable &t = u->tables[comp_in + c];
-            a.has_bc[c] = (t.any && t.heads && t.entries) ? 1 : 0;
+            a.has_bc[c] = (t.any && t.heads) ? 1 : 0;
             a.heads[c] = t.heads;
-            a.entries[c] = t.entries;
         }
     }
     for (int c = ncomp; c < kMaxComp; ++c) {
         a.has_bc[c] = 0;
         a.heads[c] = nullptr;
-        a.entries[c] = nullptr;
     }
     for (int d = 0; d < 3; ++d)
         a.ih2[d] = 1. / (u->h[d] * u->h[d]);

@@ -40,7 +40,6 @@ struct W5Args {
     int nzc, zchunk, tiles_per_comp;
     int has_bc[kWMaxComp];
     const DevBCHead *heads[kWMaxComp];
-    const DevBC *entries[kWMaxComp];
 };
 
 template <typename T, int NX, int NY, int WG>
@@ -63,8 +62,7 @@ __global__ __launch_bounds__(WG) void k_weno5(const W5Args a)
     T *ob = reinterpret_cast<T *>(a.out) + (long long)(6 * comp) * a.ocstride + blk * a.G.bstride;
 
     FaceL<T> F[6];
-    const int sb[3] = {-3, -3, -3}, se[3] = {4, 4, 4};
-    make_faces<T>(a.G, a.heads[comp], a.entries[comp], a.has_bc[comp], blk, cbase, sb, se, F);
+    make_faces<T>(a.G, a.heads[comp], a.has_bc[comp], blk, cbase, F);
     w5_march<T, NX, NY, WG>(ub, ob, a.ocstride, F, NZ, z0, z1, lds);
 }
 
@@ -81,8 +79,7 @@ __global__ __launch_bounds__(256) void k_weno5_generic(const W5Args a)
     const T *ub = cbase + blk * a.G.bstride;
     T *ob = reinterpret_cast<T *>(a.out) + (long long)(6 * comp) * a.ocstride + blk * a.G.bstride;
     FaceL<T> F[6];
-    const int sb[3] = {-3, -3, -3}, se[3] = {4, 4, 4};
-    make_faces<T>(a.G, a.heads[comp], a.entries[comp], a.has_bc[comp], blk, cbase, sb, se, F);
+    make_faces<T>(a.G, a.heads[comp], a.has_bc[comp], blk, cbase, F);
     const int *n = a.G.n;
     const long long cells = (long long)n[0] * n[1] * n[2];
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -256,15 +253,13 @@ int launch_weno5(cnv_grid_s *in, cnv_grid_s *out, hipStream_t st, const int *til
             rc = check_faces_w5(in, c);
             if (rc != CNV_OK)
                 return rc;
-            a.has_bc[c] = (in->tables[c].any && in->tables[c].heads && in->tables[c].entries) ? 1 : 0;
+            a.has_bc[c] = (in->tables[c].any && in->tables[c].heads) ? 1 : 0;
             a.heads[c] = in->tables[c].heads;
-            a.entries[c] = in->tables[c].entries;
         }
     }
     for (int c = nc; c < kWMaxComp; ++c) {
         a.has_bc[c] = 0;
         a.heads[c] = nullptr;
-        a.entries[c] = nullptr;
     }
     a.nzc = a.zchunk = a.tiles_per_comp = 0;
     W5Tune over;

@@ -20,8 +20,10 @@
 // planes loaded ahead.  FP64 grids are evaluated without contraction in the
 // operation order of the CPU restatement (bit-identical); FP32 grids let the
 // compiler fuse multiply-adds and use the hardware reciprocal.
+#include "cnv_cols.h"
 #include "cnv_march.h"
 
+#include <algorithm>
 #include <map>
 #include <type_traits>
 #include <utility>
@@ -66,54 +68,93 @@ __global__ __launch_bounds__(WG) void k_weno5(const W5Args a)
     w5_march<T, NX, NY, WG>(ub, ob, a.ocstride, F, NZ, z0, z1, lds);
 }
 
-// Generic fallback for any block shape: one thread per cell, values through
-// the resolved faces (ghost width up to 2 read, faces resolved for (-3,4)).
-template <typename T>
-__global__ __launch_bounds__(256) void k_weno5_generic(const W5Args a)
+// Blocks of any shape: a lane per VEC cells of a row and chunk of z planes
+// (cnv_cols.h), the z stencil in a register queue of planes, the two rows and
+// two cells on either side loaded per plane.  BC: some component's blocks
+// carry BC lists.  Bound by the store stream (six values per value read) and,
+// small, by load latency: 829k x 2 FP64 cells in 20x12x18 blocks 55 -> 29 us (3.2
+// TB/s of one read and six writes), 864k x 5 FP32 cells in 24^3 blocks 68 us (3.5),
+// 64 8^3 FP64 blocks 7.4; one thread per cell with 64-bit index divisions before.
+template <typename T, int VEC, bool BC>
+__global__ __launch_bounds__(kColWG) void k_weno5_cols(const W5Args a, const ColShape s)
 {
-    const long long nbt = (long long)a.G.nb[0] * a.G.nb[1] * a.G.nb[2];
-    const long long slot = blockIdx.y;
-    const int comp = (int)(slot / nbt);
-    const long long blk = slot - comp * nbt;
-    const T *cbase = reinterpret_cast<const T *>(a.in) + (long long)comp * a.G.cstride;
-    const T *ub = cbase + blk * a.G.bstride;
-    T *ob = reinterpret_cast<T *>(a.out) + (long long)(6 * comp) * a.ocstride + blk * a.G.bstride;
-    FaceL<T> F[6];
-    make_faces<T>(a.G, a.heads[comp], a.has_bc[comp], blk, cbase, F);
-    const int *n = a.G.n;
-    const long long cells = (long long)n[0] * n[1] * n[2];
-    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (i >= cells)
+    using V = VecT<T, VEC>;
+    const ColLane c = col_lane<VEC>(s, a.G);
+    if (!c.on)
         return;
-    const int x = (int)(i % n[0]);
-    const int y = (int)((i / n[0]) % n[1]);
-    const int z = (int)(i / ((long long)n[0] * n[1]));
-    const long long nx = n[0], nxy = (long long)n[0] * n[1];
-    auto at = [&](int xx, int yy, int zz) -> T {
-        if (xx < 0)
-            return face_layer(F[0], -xx, 1, nx * yy + nxy * zz);
-        if (xx >= n[0])
-            return face_layer(F[1], xx - n[0] + 1, 1, nx * yy + nxy * zz);
-        if (yy < 0)
-            return face_layer(F[2], -yy, nx, xx + nxy * zz);
-        if (yy >= n[1])
-            return face_layer(F[3], yy - n[1] + 1, nx, xx + nxy * zz);
-        if (zz < 0)
-            return face_layer(F[4], -zz, nxy, xx + nx * yy);
-        if (zz >= n[2])
-            return face_layer(F[5], zz - n[2] + 1, nxy, xx + nx * yy);
-        return ub[xx + nx * yy + nxy * zz];
+    const int nx = a.G.n[0], ny = a.G.n[1], nz = a.G.n[2];
+    const long long nxy = (long long)nx * ny;
+    const long long row = (long long)nx * c.y; // within a plane
+    const T *cb = reinterpret_cast<const T *>(a.in) + (long long)c.comp * a.G.cstride;
+    const T *ub = cb + c.blk * a.G.bstride;
+    const DevBCHead *h = nullptr;
+    if (BC && a.has_bc[c.comp])
+        h = a.heads[c.comp] + c.blk;
+    auto nbr = [&](int f) { return cb + c.nbr[f] * a.G.bstride; };
+    // cell x of this row / row y at this lane's cells / plane z of its column,
+    // up to two past the block (its plane 0 where a plane is added later)
+    auto cell = [&](int x) -> ColNb<T> {
+        if (x < 0)
+            return col_ghost<T, BC>(h, 0, nbr(0) + row + (nx + x), ub + row, ub + row + (-1 - x));
+        if (x >= nx)
+            return col_ghost<T, BC>(h, 1, nbr(1) + row + (x - nx), ub + row + (nx - 1), ub + row + (2 * nx - 1 - x));
+        return {ub + row + x, (T)1, false};
     };
-    T um, up;
-    weno5<T>(at(x - 2, y, z), at(x - 1, y, z), ub[i], at(x + 1, y, z), at(x + 2, y, z), um, up);
-    ob[i] = um;
-    ob[a.ocstride + i] = up;
-    weno5<T>(at(x, y - 2, z), at(x, y - 1, z), ub[i], at(x, y + 1, z), at(x, y + 2, z), um, up);
-    ob[2 * a.ocstride + i] = um;
-    ob[3 * a.ocstride + i] = up;
-    weno5<T>(at(x, y, z - 2), at(x, y, z - 1), ub[i], at(x, y, z + 1), at(x, y, z + 2), um, up);
-    ob[4 * a.ocstride + i] = um;
-    ob[5 * a.ocstride + i] = up;
+    auto line = [&](int y) -> ColNb<T> {
+        const T *x0 = ub + c.x0;
+        if (y < 0)
+            return col_ghost<T, BC>(h, 2, nbr(2) + c.x0 + (long long)nx * (ny + y), x0, x0 + (long long)nx * (-1 - y));
+        if (y >= ny)
+            return col_ghost<T, BC>(h, 3, nbr(3) + c.x0 + (long long)nx * (y - ny), x0 + (long long)nx * (ny - 1),
+                                    x0 + (long long)nx * (2 * ny - 1 - y));
+        return {x0 + (long long)nx * y, (T)1, false};
+    };
+    const T *col = ub + row + c.x0;
+    auto plane = [&](int z) -> V {
+        if (z < 0)
+            return col_load<T, VEC, BC>(col_ghost<T, BC>(h, 4, nbr(4) + row + c.x0 + nxy * (nz + z), col,
+                                                         col + nxy * (-1 - z)), 0);
+        if (z >= nz)
+            return col_load<T, VEC, BC>(col_ghost<T, BC>(h, 5, nbr(5) + row + c.x0 + nxy * (z - nz),
+                                                         col + nxy * (nz - 1), col + nxy * (2 * nz - 1 - z)), 0);
+        return load_vec<T, VEC>(col + nxy * z);
+    };
+    const ColNb<T> xa = cell(c.x0 - 2), xb = cell(c.x0 - 1), xd = cell(c.x0 + VEC), xe = cell(c.x0 + VEC + 1);
+    const ColNb<T> ya = line(c.y - 2), yb = line(c.y - 1), yd = line(c.y + 1), ye = line(c.y + 2);
+    T *ob = reinterpret_cast<T *>(a.out) + (long long)(6 * c.comp) * a.ocstride + c.blk * a.G.bstride + row + c.x0;
+    V q0 = plane(c.z0 - 2), q1 = plane(c.z0 - 1), q2 = plane(c.z0), q3 = plane(c.z0 + 1), q4 = plane(c.z0 + 2);
+    for (int z = c.z0; z < c.z1; ++z) {
+        const long long o = nxy * z;
+        // x: the row's cells and two on either side
+        T xs[VEC + 4];
+        xs[0] = col_load1<T, BC>(xa, o);
+        xs[1] = col_load1<T, BC>(xb, o);
+        xs[VEC + 2] = col_load1<T, BC>(xd, o);
+        xs[VEC + 3] = col_load1<T, BC>(xe, o);
+        const V va = col_load<T, VEC, BC>(ya, o), vb = col_load<T, VEC, BC>(yb, o);
+        const V vd = col_load<T, VEC, BC>(yd, o), ve = col_load<T, VEC, BC>(ye, o);
+        V q5 = q4;
+        if (z + 1 < c.z1)
+            q5 = plane(z + 3);
+#pragma unroll
+        for (int v = 0; v < VEC; ++v)
+            xs[v + 2] = q2.v[v];
+        V r[6];
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) {
+            weno5<T>(q0.v[v], q1.v[v], q2.v[v], q3.v[v], q4.v[v], r[4].v[v], r[5].v[v]);
+            weno5<T>(xs[v], xs[v + 1], xs[v + 2], xs[v + 3], xs[v + 4], r[0].v[v], r[1].v[v]);
+            weno5<T>(va.v[v], vb.v[v], q2.v[v], vd.v[v], ve.v[v], r[2].v[v], r[3].v[v]);
+        }
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+            store_nt<T, VEC>(ob + k * a.ocstride + o, r[k]);
+        q0 = q1;
+        q1 = q2;
+        q2 = q3;
+        q3 = q4;
+        q4 = q5;
+    }
 }
 
 // ---------------------------------------------------------------- host side
@@ -134,11 +175,48 @@ static W5Tune w5_default(int dtype, int edge)
     return W5Tune{256, 16};
 }
 
-static W5Tune w5_tune(int dtype, int edge)
+// pinned: set to something else than the built-in tile
+static W5Tune w5_tune(int dtype, int edge, bool *pinned = nullptr)
 {
     std::lock_guard<std::mutex> lk(g_w5_mtx);
     auto it = g_w5_tune.find({dtype, edge});
-    return it == g_w5_tune.end() ? w5_default(dtype, edge) : it->second;
+    const W5Tune d = w5_default(dtype, edge), t = it == g_w5_tune.end() ? d : it->second;
+    if (pinned)
+        *pinned = t.wg != d.wg || t.zchunk != d.zchunk;
+    return t;
+}
+
+// The tile of a launch over `nbc` blocks times components of nz planes: the
+// pinned one, else the built-in one with the deepest z chunk (down to two
+// planes) that gives enough tiles to fill the GPU.  A chunk's planes run one
+// after another, about 2 us each, so on a grid of few tiles the chain is the
+// launch.  Built-in depth / this rule: 128^3 FP32 in 32^3 blocks 68.8 / 18.8 us,
+// in 64^3 blocks 107 / 20.7, 192^3 FP64 in 32^3 blocks 116 / 91, 256^3 FP32 in
+// 64^3 blocks 124 / 103; twice or half as many tiles: 20.6 and 23.3, 31.9 (half),
+// 99 and 116, 118 and 124.
+static W5Tune w5_tile(int dtype, int edge, long long nbc, int nz)
+{
+    bool pinned = false;
+    W5Tune t = w5_tune(dtype, edge, &pinned);
+    if (pinned)
+        return t;
+    const long long enough =
+        edge >= 64 ? (dtype == CNV_F64 ? 200 : 400) : edge == 32 ? 400 : dtype == CNV_F64 ? 800 : 1500;
+    auto tiles = [&](int z) { return nbc * ((nz + z - 1) / z); };
+    t.zchunk = std::min(t.zchunk, nz);
+    while (t.zchunk > 2 && tiles(t.zchunk) < enough)
+        t.zchunk = (t.zchunk + 1) / 2;
+    return t;
+}
+
+// Grids of 16, 32 or 64 cells per x/y edge run as columns below 1.2M cells
+// times components unless a tile is pinned: 32^3 FP32 69 -> 7.1 us, 64^3 FP64 in
+// 32^3 blocks 93 -> 9.4, 96^3 FP64 in 16^3 blocks 32.5 -> 20.4.  At 2.1M cells the
+// marching tile of the rule above is level or ahead (18.8 / 20.8 us FP32, 30.0 /
+// 31.0 FP64 in 32^3 blocks).
+static bool w5_cols_for_small(const Geom &G, int ncomp)
+{
+    return (long long)G.nb[0] * G.nb[1] * G.nb[2] * ncomp * G.n[0] * G.n[1] * G.n[2] < 1200000;
 }
 
 template <typename T, int NX, int WG>
@@ -174,13 +252,59 @@ static bool w5_dispatch_wg(const W5Args &a, int wg, int ntiles, hipStream_t st)
     }
 }
 
+// The column kernel on blocks of any shape.
+template <typename T>
+static int w5_cols(const W5Args &a, hipStream_t st)
+{
+    const int *n = a.G.n;
+    const long long gx = ((long long)n[0] * n[1] * n[2] + 255) / 256;
+    const long long gy = (long long)a.G.nb[0] * a.G.nb[1] * a.G.nb[2] * a.ncomp;
+    if (gx > 0x7fffffffLL || gy > 65535)
+        return fail(CNV_ERR_UNSUPPORTED, "grid too large for the generic WENO5 kernel");
+    const int vec = col_vec(n[0], sizeof(T));
+    // planes per lane: FP64 as many as leave the two and a half waves per SIMD
+    // that its registers allow at once, FP32 two and a half times as many lanes;
+    // 16 at most.  24^3 x 5 FP32 68 us with 450k lanes, 78 with 180k; 48^3 x 2
+    // FP32 60 with 500k, 70 with 166k; 20x12x18 x 2 FP64 29 with 184k, 32 with 276k
+    // and 138k.
+    const long long vectors = gy * ((long long)n[0] / vec * n[1] * n[2]);
+    const int z = (int)std::min<long long>(16, std::max<long long>(1, vectors / (sizeof(T) == 4 ? 409600 : 163840)));
+    ColShape s;
+    long long nwg = 0;
+    if (!col_shape(a.G, a.ncomp, vec, std::min(z, n[2]), s, nwg))
+        return fail(CNV_ERR_UNSUPPORTED, "grid too large for the generic WENO5 kernel");
+    bool bc = false;
+    for (int c = 0; c < a.ncomp; ++c)
+        bc = bc || a.has_bc[c];
+    auto go = [&](auto v) {
+        constexpr int VEC = decltype(v)::value;
+        if (bc)
+            hipLaunchKernelGGL((k_weno5_cols<T, VEC, true>), dim3((unsigned)nwg), dim3(kColWG), 0, st, a, s);
+        else
+            hipLaunchKernelGGL((k_weno5_cols<T, VEC, false>), dim3((unsigned)nwg), dim3(kColWG), 0, st, a, s);
+    };
+    if (vec == 1)
+        go(std::integral_constant<int, 1>());
+    else if (vec == 2)
+        go(std::integral_constant<int, 2>());
+    else if constexpr (sizeof(T) == 4)
+        go(std::integral_constant<int, 4>());
+    CNV_HIP(hipGetLastError());
+    return CNV_OK;
+}
+
 template <typename T>
 static int w5_run(W5Args &a, hipStream_t st, const W5Tune *over)
 {
     const int *n = a.G.n;
     const long long nbt = (long long)a.G.nb[0] * a.G.nb[1] * a.G.nb[2];
     if (n[0] == n[1] && (n[0] == 16 || n[0] == 32 || n[0] == 64)) {
-        const W5Tune tu = over ? *over : w5_tune(sizeof(T) == 8 ? CNV_F64 : CNV_F32, n[0]);
+        const int dtype = sizeof(T) == 8 ? CNV_F64 : CNV_F32;
+        bool pinned = false;
+        (void)w5_tune(dtype, n[0], &pinned);
+        if (!over && !pinned && w5_cols_for_small(a.G, a.ncomp))
+            return w5_cols<T>(a, st);
+        const W5Tune tu = over ? *over : w5_tile(dtype, n[0], nbt * a.ncomp, n[2]);
         a.zchunk = tu.zchunk < n[2] ? tu.zchunk : n[2];
         a.nzc = (n[2] + a.zchunk - 1) / a.zchunk;
         a.tiles_per_comp = (int)(nbt * a.nzc);
@@ -201,13 +325,7 @@ static int w5_run(W5Args &a, hipStream_t st, const W5Tune *over)
         if (over)
             return fail(CNV_ERR_UNSUPPORTED, "tile shape not available for this block edge and dtype");
     }
-    const long long cells = (long long)n[0] * n[1] * n[2];
-    const long long gx = (cells + 255) / 256, gy = nbt * a.ncomp;
-    if (gx > 0x7fffffffLL || gy > 65535)
-        return fail(CNV_ERR_UNSUPPORTED, "grid too large for the generic WENO5 kernel");
-    hipLaunchKernelGGL(k_weno5_generic<T>, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, st, a);
-    CNV_HIP(hipGetLastError());
-    return CNV_OK;
+    return w5_cols<T>(a, st);
 }
 
 static int check_faces_w5(cnv_grid_s *g, int comp)

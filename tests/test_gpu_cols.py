@@ -100,3 +100,28 @@ def test_run_depth_by_grid_size(gpu, dtype, nb, edge):
     assert_same(res.download(0), a.download(0))
     gn, wn = norms.download(np.float64, 6), want.download(np.float64, 6)
     assert np.max(np.abs(gn - wn) / wn) <= 1e-13
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("shape", [x for x in SHAPES if min(x[1]) >= 2] + [((2, 1, 1), (2, 3, 2)), ((1, 2, 1), (3, 2, 17))],
+                         ids=str)
+@pytest.mark.parametrize("lists", [[[]], [MIXED, [], PARTLY]], ids=["periodic", "walls"])
+def test_weno5_columns(gpu, dtype, shape, lists):
+    """FP64: the oracle's bits.  FP32: the oracle's FP32 evaluation divides where
+    the kernel multiplies by hardware reciprocals (1 ulp each, three per
+    state), so a few ulp of the stencil's largest value."""
+    nb, n = shape
+    g, slabs, bcs = build(nb, n, dtype, 23, lists)
+    out = cnv.Cartesian(nb, n, dtype=dtype, ncomp=6 * len(lists))
+    cnv.weno5(g, out)
+    for c, slab in enumerate(slabs):
+        f = oracle.Field(slab.astype(np.float64), nb, n, g.block_stride, bcs=bcs[c])
+        want = oracle.weno5(f, prec=1)
+        for k in range(6):
+            got = cells_of(out.download(6 * c + k), nb, n, g.block_stride)
+            ref = cells_of(want[k], nb, n, g.block_stride)
+            if dtype is np.float64:
+                assert_same(got, ref, "comp %d state %d" % (c, k))
+            else:
+                assert np.max(np.abs(got - ref)) <= 1e-5 * np.max(np.abs(slab))
+                assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)

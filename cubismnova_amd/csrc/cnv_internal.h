@@ -216,13 +216,32 @@ int launch_diffusion_noalloc(const cnv_grid_desc *desc, const void *u, void *u_n
 
 int launch_sums(cnv_grid_s *g, int comp, double *out, hipStream_t st);
 int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_dt, double *norms, hipStream_t st);
-// two Euler steps per launch on periodic grids (cnv_stencil7x2.hip)
+// Rule of a domain face as the two-step and two-sweep kernels apply it to the
+// ghost cells they read past it: the periodic neighbour, a constant
+// (Dirichlet, BC/Dirichlet.h:75-113), sign times the mirror cell (Symmetry,
+// BC/Symmetry.h:69-114: ghost layer l reads interior cell l - 1 from the
+// face), or the face's own cell (Absorbing, BC/Absorbing.h:66-105: every
+// layer reads interior cell 0 from the face).
+enum { FM_PERIODIC = 0, FM_CONST = 1, FM_MIRROR = 2, FM_EDGE = 3 };
+// the six rules of a component; false unless every domain face has one rule on
+// all its blocks and every inner face is a neighbour copy (cnv_jacobi2.hip)
+bool jacobi2_faces(cnv_grid_s *g, int comp, int fm[3][2], double fv[3][2]);
+
+// two Euler steps per launch on periodic grids, and on grids with walls with
+// the faces of every component (cnv_stencil7x2.hip)
+constexpr int kX2MaxComp = 8;
+struct X2Faces {
+    int fm[3][2];
+    double fv[3][2];
+};
+
+bool x2_walls(cnv_grid_s *u, X2Faces *faces);
 bool x2_applicable(cnv_grid_s *u);
 long long x2_tiles(const cnv_grid_s *u, int zchunk);
 void x2_tile(cnv_grid_s *u, int *wg, int *zchunk);
 int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *part1, double *part2,
                         const double *const prev_p[2], const int prev_n[2], double *const prev_out[2], int wg,
-                        int zchunk, int *nparts, hipStream_t st);
+                        int zchunk, int *nparts, hipStream_t st, const X2Faces *faces = nullptr);
 int x2_set_tune(int dtype, int edge, int wg, int zchunk);
 int x2_get_tune(int dtype, int edge, int *wg, int *zchunk);
 int autotune_x2(cnv_grid_s *u, cnv_grid_s *out, int iters, int *best_wg, int *best_z, double *results,

@@ -27,14 +27,6 @@ namespace cnv
 
 constexpr int kJ2ZMax = 64; // planes per tile at most
 
-// Rule of a domain face as the two-sweep kernel applies it to the ghost
-// cells the sweeps read past it: the periodic neighbour, a constant
-// (Dirichlet, BC/Dirichlet.h:75-113), sign times the mirror cell (Symmetry,
-// BC/Symmetry.h:69-114: ghost layer l reads interior cell l - 1 from the
-// face), or the face's own cell (Absorbing, BC/Absorbing.h:66-105: every
-// layer reads interior cell 0 from the face).
-enum { FM_PERIODIC = 0, FM_CONST = 1, FM_MIRROR = 2, FM_EDGE = 3 };
-
 struct J2Args {
     const char *u;  // grid base of u (component cu)
     const char *f;  // grid base of f (component cf)

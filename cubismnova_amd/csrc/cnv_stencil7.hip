@@ -640,8 +640,8 @@ int launch_diffusion_noalloc(const cnv_grid_desc *desc, const void *u, void *u_n
     return launch_stencil7_t(&gu, &go, nullptr, 0, 0, desc->ncomp, 1, nu_dt, sumsq, st, nullptr, nullptr, &scr);
 }
 
-// nsteps Euler steps alternating u -> tmp -> u ...  On periodic grids of
-// 16^3 or 32^3 blocks an even number of two-step launches covers the steps
+// nsteps Euler steps alternating u -> tmp -> u ...  On grids of 16^3 or 32^3
+// blocks that are periodic or have walls of one rule each an even number of two-step launches covers the steps
 // up to a multiple of four, single steps the rest (so the field ends in u
 // for even nsteps, in tmp for odd).  The norms of a launch are reduced by
 // workgroup 0 of the next launch from the other half of u's partial buffer,
@@ -651,7 +651,10 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
     double *P[2] = {u->partials, u->partials + u->partials_cap};
     const size_t cap = u->partials_cap;
     int nfused = 0, xwg = 0, xz = 0;
-    if (nsteps >= 4 && !force_generic() && x2_applicable(u) && x2_applicable(tmp)) {
+    X2Faces faces[kX2MaxComp];
+    const bool periodic = nsteps >= 4 && !force_generic() && x2_applicable(u) && x2_applicable(tmp);
+    const bool walls = nsteps >= 4 && !force_generic() && !periodic && x2_walls(u, faces);
+    if (periodic || walls) {
         x2_tile(u, &xwg, &xz);
         if (2 * x2_tiles(u, xz) <= (long long)cap)
             nfused = 2 * (nsteps / 4);
@@ -666,7 +669,7 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
         double *p2 = norms ? p1 + x2_tiles(u, xz) : nullptr;
         int nt = 0;
         const int rc = launch_diffusion_x2(grid_at(L), grid_at(L + 1), nu_dt, p1, p2, prev, prev_n, prev_out, xwg, xz,
-                                           &nt, st);
+                                           &nt, st, walls ? faces : nullptr);
         if (rc != CNV_OK)
             return rc;
         if (norms) {

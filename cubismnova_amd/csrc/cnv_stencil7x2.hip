@@ -1,5 +1,6 @@
 // cnv_stencil7x2.hip -- two forward-Euler diffusion steps per launch on
-// periodic grids (every face of every block a neighbour copy, no BC list).
+// periodic grids (every face of every block a neighbour copy, no BC list) and
+// on grids whose domain faces are walls of one rule each.
 //
 // A workgroup owns the x-y planes [z0, z1) of one block of one component.
 // It stages the planes of u^n it needs, each with a two-cell x/y halo from
@@ -34,6 +35,7 @@ struct X2Args {
     const double *prev_p[2];
     int prev_n[2];
     double *prev_out[2];
+    X2Faces faces[kX2MaxComp]; // WALL kernels only
 };
 
 template <typename T, int N, int WG>
@@ -87,7 +89,16 @@ constexpr int kDppRowShl1 = 0x101; // lane i <- lane i+1
 
 // ZC planes per tile: the ZC + 2 planes of u^{n+1} run as a static rotation
 // of the three register slots, so every slot index is a constant.
-template <typename T, int N, int WG, int ZC>
+//
+// WALL: some domain face is no periodic neighbour copy.  A ghost past a wall is
+// the face's constant, or its factor times the cell next to the wall (the
+// mirror of layer 1 and the edge cell are that cell), for u^n as for u^{n+1};
+// layer 2 past a wall is never read, because no u^{n+1} is evaluated past one.
+// The thread that evaluates the cell next to a mirror or edge wall also writes
+// its ghost.  41 FP64 steps of 192x160x128 cells in 32^3 blocks between walls 728
+// -> 432 us against one step per launch; per step 256^3 17.0 us FP32, 29.9 FP64
+// (periodic 15.2 and 26.1: the wall rules cost 12-25 % in instructions).
+template <typename T, int N, int WG, int ZC, bool WALL>
 __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
 {
     using S = X2Shape<T, N, WG>;
@@ -141,32 +152,93 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
     // plane offset.
     unsigned hsrc[HS]; // byte offset within the source plane's z-layer of blocks
     int hlds[HS], hkind[HS];
+    // WALL: the value read, times hm, or the constant hv past a Dirichlet wall
+    T hm[HS], hv[HS];
+    bool hc[HS];
+    const X2Faces &fc = a.faces[WALL ? comp : 0];
+    // cell l of block b along axis d (l = -2 .. N + 1) as (block, cell) of the
+    // source; past a wall the cell next to it and the wall's rule
+    struct Src {
+        int b, l;
+        T m, v;
+        bool cst;
+    };
+    auto source = [&](int d, int b, int nb, int l) __attribute__((always_inline)) -> Src {
+        const int side = l >= N;
+        Src r{b, l, (T)1, (T)0, false};
+        if (l >= 0 && l < N)
+            return r;
+        const int rule = WALL && (side ? b == nb - 1 : b == 0) ? fc.fm[d][side] : FM_PERIODIC;
+        if (rule == FM_PERIODIC) {
+            r.b = wrap(b + (side ? 1 : -1), nb);
+            r.l = side ? l - N : l + N;
+            return r;
+        }
+        const T f = (T)fc.fv[d][side];
+        r.l = side ? N - 1 : 0;
+        r.cst = rule == FM_CONST;
+        r.v = f;
+        r.m = rule == FM_MIRROR ? f : (T)1;
+        return r;
+    };
 #pragma unroll
     for (int h = 0; h < HS; ++h) {
         const int s = tid + h * WG;
-        hkind[h] = 0;
-        hsrc[h] = 0;
-        hlds[h] = 0;
+        int x = 0, y = 0, kind = 0;
         if (s < NHX) {
-            const int side = s / (2 * N), lyr = (s / N) & 1, y = s % N;
-            const long long nb = (wrap(bx + (side ? 1 : -1), nbx) + (long long)nbx * by) * bstride;
-            hsrc[h] = (unsigned)((nb + (side ? lyr : N - 1 - lyr) + N * y) * TS);
-            hlds[h] = (y + 2) * PA + VEC + (side ? N + lyr : -1 - lyr);
-            hkind[h] = 1;
+            const int side = s / (2 * N), lyr = (s / N) & 1;
+            x = side ? N + lyr : -1 - lyr;
+            y = s % N;
+            kind = 1;
         } else if (s < NHX + NHY) {
             const int s2 = s - NHX;
-            const int side = s2 / (2 * TX), lyr = (s2 / TX) & 1, xs = (s2 % TX) * VEC;
-            const long long nb = (bx + (long long)nbx * wrap(by + (side ? 1 : -1), nby)) * bstride;
-            hsrc[h] = (unsigned)((nb + xs + N * (side ? lyr : N - 1 - lyr)) * TS);
-            hlds[h] = ((side ? N + lyr : -1 - lyr) + 2) * PA + VEC + xs;
-            hkind[h] = 2;
+            const int side = s2 / (2 * TX), lyr = (s2 / TX) & 1;
+            x = (s2 % TX) * VEC;
+            y = side ? N + lyr : -1 - lyr;
+            kind = 2;
         } else if (s < NH) {
-            const int d = s - NHX - NHY, sx = d & 1, sy = d >> 1;
-            const long long nb =
-                (wrap(bx + (sx ? 1 : -1), nbx) + (long long)nbx * wrap(by + (sy ? 1 : -1), nby)) * bstride;
-            hsrc[h] = (unsigned)((nb + (sx ? 0 : N - 1) + N * (sy ? 0 : N - 1)) * TS);
-            hlds[h] = ((sy ? N : -1) + 2) * PA + VEC + (sx ? N : -1);
-            hkind[h] = 1;
+            const int d = s - NHX - NHY;
+            x = (d & 1) ? N : -1;
+            y = (d >> 1) ? N : -1;
+            kind = 1;
+        }
+        const Src sx = source(0, bx, nbx, x), sy = source(1, by, nby, y);
+        hsrc[h] = (unsigned)(((sx.b + (long long)nbx * sy.b) * bstride + sx.l + N * sy.l) * TS);
+        hlds[h] = (y + 2) * PA + VEC + x;
+        hkind[h] = kind;
+        hm[h] = sx.m * sy.m; // one of them is 1 wherever the value is used
+        hv[h] = sx.cst ? sx.v : sy.v;
+        hc[h] = sx.cst || sy.cst;
+    }
+    // WALL: ring cells past a wall: a constant (1), or written by the thread
+    // of the cell next to it (2); the factors of this thread's cells next to
+    // a mirror or edge wall (0: none) and of the z walls
+    int rk[RS];
+    T rv[RS];
+    T gx0 = (T)0, gx1 = (T)0, gy0 = (T)0, gy1 = (T)0, gz0 = (T)0, gz1 = (T)0;
+    if constexpr (WALL) {
+        auto past = [&](int d, int side, int b, int nb) { // rule past this side of the block, 0: a neighbour
+            return (side ? b == nb - 1 : b == 0) ? fc.fm[d][side] : FM_PERIODIC;
+        };
+        auto factor = [&](int d, int side, int b, int nb) -> T {
+            const int k = past(d, side, b, nb);
+            return k == FM_MIRROR ? (T)fc.fv[d][side] : k == FM_EDGE ? (T)1 : (T)0;
+        };
+        if (x0 == 0)
+            gx0 = factor(0, 0, bx, nbx);
+        if (x0 + VEC == N)
+            gx1 = factor(0, 1, bx, nbx);
+        gy0 = factor(1, 0, by, nby);
+        gy1 = factor(1, 1, by, nby);
+        gz0 = factor(2, 0, bz, nbz);
+        gz1 = factor(2, 1, bz, nbz);
+#pragma unroll
+        for (int h = 0; h < RS; ++h) {
+            const int s = tid + h * WG;
+            const int d = s < 2 * N ? 0 : 1, side = (s / N) & 1;
+            const int k = d == 0 ? past(0, side, bx, nbx) : past(1, side, by, nby);
+            rk[h] = k == FM_PERIODIC ? 0 : k == FM_CONST ? 1 : 2;
+            rv[h] = (T)fc.fv[d][side];
         }
     }
     const int own = x0 + N * ty; // this thread's first row offset within a plane
@@ -176,11 +248,11 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
         V h[HS];
     };
     // plane p (z0-2 <= p <= z1+1, possibly in the z-neighbour block) into registers
-    auto load_u0 = [&](int p) -> U0 {
+    auto load_u0 = [&](int p) __attribute__((always_inline)) -> U0 {
         U0 Q; // scalar halo entries use element 0 only
-        const int dz = p < 0 ? -1 : (p >= N ? 1 : 0);
+        const Src sz = source(2, bz, nbz, p);
         // byte offset of plane p of this block row's z-layer (uniform)
-        const unsigned lb = (unsigned)(((long long)wrap(bz + dz, nbz) * layer + (long long)(p - dz * N) * NN) * TS);
+        const unsigned lb = (unsigned)((sz.b * layer + (long long)sz.l * NN) * TS);
         const unsigned sb = lb + (unsigned)(xyself * TS);
 #pragma unroll
         for (int r = 0; r < R; ++r)
@@ -192,6 +264,22 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
             } else if (hkind[h] == 1) {
                 Q.h[h].v[0] = buf_load1<T>(rin, hsrc[h], lb);
             }
+        }
+        if constexpr (WALL) {
+            // (uniform: only planes past a z wall)
+            if (sz.cst || sz.m != (T)1) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int v = 0; v < VEC; ++v)
+                        Q.c[r].v[v] = sz.cst ? sz.v : sz.m * Q.c[r].v[v];
+            }
+#pragma unroll
+            for (int h = 0; h < HS; ++h)
+#pragma unroll
+                for (int v = 0; v < VEC; ++v)
+                    if (v == 0 || hkind[h] == 2)
+                        Q.h[h].v[v] = sz.cst ? sz.v : hc[h] ? hv[h] : sz.m * (hm[h] * Q.h[h].v[v]);
         }
         return Q;
     };
@@ -298,8 +386,28 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
                 res.v[v] = euler(c0c[r].v[v], xm, xp, ym.v[v], yp.v[v], c0m[r].v[v], c0p[r].v[v]);
             }
             n1[r] = res;
-            if (inner)
+            if (inner) {
                 *reinterpret_cast<V *>(Bq + (y + 1) * PA + VEC + x0) = res;
+                if constexpr (WALL) { // ghosts of u^{n+1} past mirror and edge walls
+                    if (gx0 != (T)0)
+                        Bq[(y + 1) * PA + VEC - 1] = gx0 * res.v[0];
+                    if (gx1 != (T)0)
+                        Bq[(y + 1) * PA + VEC + N] = gx1 * res.v[VEC - 1];
+                    if ((y == 0 && gy0 != (T)0) || (y == N - 1 && gy1 != (T)0)) {
+                        V g;
+#pragma unroll
+                        for (int v = 0; v < VEC; ++v)
+                            g.v[v] = (y == 0 ? gy0 : gy1) * res.v[v];
+                        *reinterpret_cast<V *>(Bq + (y == 0 ? 0 : N + 1) * PA + VEC + x0) = g;
+                    }
+                }
+            } else if constexpr (WALL) { // a plane past a Dirichlet z wall keeps its constant
+                const int side = q >= N;
+                if ((q < 0 || q >= N) && fc.fm[2][side] == FM_CONST && (side ? bz == nbz - 1 : bz == 0))
+#pragma unroll
+                    for (int v = 0; v < VEC; ++v)
+                        n1[r].v[v] = (T)fc.fv[2][side];
+            }
         }
         // plane q - 1 has served: the next u^n plane goes into its slot
         if (q + 2 <= z1 + 1) {
@@ -330,9 +438,11 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
                     rz[(u + 2) % 3][h] = Ap[o];
                     if (q == z0 - 1)
                         rz[(u + 1) % 3][h] = Ac[o];
-                    if (inner)
-                        Bq[(y + 1) * PA + VEC + x] = euler(rz[(u + 1) % 3][h], Ac[o - 1], Ac[o + 1], Ac[o - PA],
-                                                           Ac[o + PA], rz[u % 3][h], rz[(u + 2) % 3][h]);
+                    if (inner && (!WALL || rk[h] != 2)) {
+                        const T e = euler(rz[(u + 1) % 3][h], Ac[o - 1], Ac[o + 1], Ac[o - PA], Ac[o + PA],
+                                          rz[u % 3][h], rz[(u + 2) % 3][h]);
+                        Bq[(y + 1) * PA + VEC + x] = WALL && rk[h] == 1 ? rv[h] : e;
+                    }
                 }
             }
         }
@@ -358,7 +468,14 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
                 for (int v = 0; v < VEC; ++v) {
                     const T xm = v == 0 ? xl : c1[r].v[v - 1];
                     const T xp = v == VEC - 1 ? xr : c1[r].v[v + 1];
-                    res.v[v] = euler(c1[r].v[v], xm, xp, ym.v[v], yp.v[v], m1[r].v[v], n1[r].v[v]);
+                    T zm = m1[r].v[v], zp = n1[r].v[v];
+                    if constexpr (WALL) {
+                        if (q - 1 == 0 && gz0 != (T)0)
+                            zm = gz0 * c1[r].v[v];
+                        if (q - 1 == N - 1 && gz1 != (T)0)
+                            zp = gz1 * c1[r].v[v];
+                    }
+                    res.v[v] = euler(c1[r].v[v], xm, xp, ym.v[v], yp.v[v], zm, zp);
                     acc1 = __builtin_fma((double)c1[r].v[v], (double)c1[r].v[v], acc1);
                     acc2 = __builtin_fma((double)res.v[v], (double)res.v[v], acc2);
                 }
@@ -443,25 +560,27 @@ int x2_enough(int dtype, int edge)
 // chunks of 2 and 4 planes are compiled for small grids
 inline bool x2_zchunk_ok(int zc) { return zc == 8 || zc == 16 || zc == 32; }
 
-template <typename T, int N, int WG>
+template <typename T, int N, int WG, bool WALL>
 bool x2_launch1(const X2Args &a, int zc, int ntiles, hipStream_t st)
 {
     if constexpr (X2Shape<T, N, WG>::valid) {
-        if (zc == 16)
-            hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 16>), dim3(ntiles), dim3(WG), 0, st, a);
-        else if (zc == 8)
-            hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 8>), dim3(ntiles), dim3(WG), 0, st, a);
-        else if (zc == 4)
-            hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 4>), dim3(ntiles), dim3(WG), 0, st, a);
-        else if (zc == 2)
-            hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 2>), dim3(ntiles), dim3(WG), 0, st, a);
-        else if constexpr (N == 32) {
-            if (zc != 32)
-                return false;
-            hipLaunchKernelGGL((k_stencil7x2<T, N, WG, 32>), dim3(ntiles), dim3(WG), 0, st, a);
-        } else
-            return false;
-        return true;
+        auto go = [&](auto z) {
+            hipLaunchKernelGGL((k_stencil7x2<T, N, WG, decltype(z)::value, WALL>), dim3(ntiles), dim3(WG), 0, st, a);
+            return true;
+        };
+        switch (zc) {
+        case 2:
+            return go(std::integral_constant<int, 2>());
+        case 4:
+            return go(std::integral_constant<int, 4>());
+        case 8:
+            return go(std::integral_constant<int, 8>());
+        case 16:
+            return go(std::integral_constant<int, 16>());
+        case 32:
+            if constexpr (N == 32)
+                return go(std::integral_constant<int, 32>());
+        }
     }
     return false;
 }
@@ -471,13 +590,13 @@ bool x2_dispatch_wg(const X2Args &a, int wg, int zc, int ntiles, hipStream_t st)
 {
     switch (wg) {
     case 64:
-        return x2_launch1<T, N, 64>(a, zc, ntiles, st);
+        return x2_launch1<T, N, 64, false>(a, zc, ntiles, st);
     case 128:
-        return x2_launch1<T, N, 128>(a, zc, ntiles, st);
+        return x2_launch1<T, N, 128, false>(a, zc, ntiles, st);
     case 256:
-        return x2_launch1<T, N, 256>(a, zc, ntiles, st);
+        return x2_launch1<T, N, 256, false>(a, zc, ntiles, st);
     case 512:
-        return x2_launch1<T, N, 512>(a, zc, ntiles, st);
+        return x2_launch1<T, N, 512, false>(a, zc, ntiles, st);
     }
     return false;
 }
@@ -505,6 +624,16 @@ bool x2_valid(int dtype, int edge, int wg)
     return edge == 16 ? x2_valid_wg<float, 16>(wg) : x2_valid_wg<float, 32>(wg);
 }
 
+// Grids with walls run the built-in workgroup sizes.
+bool x2_dispatch_wall(int dtype, int edge, int zc, const X2Args &a, int ntiles, hipStream_t st)
+{
+    if (dtype == CNV_F64)
+        return edge == 16 ? x2_launch1<double, 16, 128, true>(a, zc, ntiles, st)
+                          : x2_launch1<double, 32, 256, true>(a, zc, ntiles, st);
+    return edge == 16 ? x2_launch1<float, 16, 64, true>(a, zc, ntiles, st)
+                      : x2_launch1<float, 32, 256, true>(a, zc, ntiles, st);
+}
+
 bool x2_dispatch(int dtype, int edge, int wg, int zc, const X2Args &a, int ntiles, hipStream_t st)
 {
     if (dtype == CNV_F64)
@@ -516,13 +645,28 @@ bool x2_dispatch(int dtype, int edge, int wg, int zc, const X2Args &a, int ntile
 
 } // namespace
 
-bool x2_applicable(cnv_grid_s *u)
+static bool x2_shape_ok(const cnv_grid_s *u)
 {
     const int *n = u->desc.block_cells;
-    if (!(n[0] == n[1] && n[1] == n[2] && (n[0] == 16 || n[0] == 32)))
-        return false;
     // the kernel addresses a component slab with 32-bit byte offsets
-    if (u->component_bytes >= ((size_t)1 << 31))
+    return n[0] == n[1] && n[1] == n[2] && (n[0] == 16 || n[0] == 32) && u->component_bytes < ((size_t)1 << 31);
+}
+
+// The faces of every component of a grid with walls, each domain face of one
+// rule on all its blocks; false for other grids (they step one at a time).
+bool x2_walls(cnv_grid_s *u, X2Faces *faces)
+{
+    if (!x2_shape_ok(u) || u->desc.ncomp > kX2MaxComp)
+        return false;
+    for (int c = 0; c < u->desc.ncomp; ++c)
+        if (!jacobi2_faces(u, c, faces[c].fm, faces[c].fv))
+            return false;
+    return true;
+}
+
+bool x2_applicable(cnv_grid_s *u)
+{
+    if (!x2_shape_ok(u))
         return false;
     std::lock_guard<std::mutex> lk(u->mtx);
     for (int c = 0; c < u->desc.ncomp; ++c)
@@ -541,7 +685,7 @@ long long x2_tiles(const cnv_grid_s *u, int zchunk)
 
 int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *part1, double *part2,
                         const double *const prev_p[2], const int prev_n[2], double *const prev_out[2], int wg,
-                        int zchunk, int *nparts, hipStream_t st)
+                        int zchunk, int *nparts, hipStream_t st, const X2Faces *faces)
 {
     const int edge = u->desc.block_cells[0];
     if (wg <= 0 || zchunk <= 0) {
@@ -572,7 +716,10 @@ int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *pa
     const long long ntiles = (long long)a.tiles_per_comp * u->desc.ncomp;
     if (ntiles >= (1LL << 31))
         return fail(CNV_ERR_UNSUPPORTED, "grid too large for the two-step kernel");
-    if (!x2_dispatch(u->desc.dtype, edge, wg, zchunk, a, (int)ntiles, st))
+    for (int c = 0; faces && c < u->desc.ncomp; ++c)
+        a.faces[c] = faces[c];
+    if (!(faces ? x2_dispatch_wall(u->desc.dtype, edge, zchunk, a, (int)ntiles, st)
+                : x2_dispatch(u->desc.dtype, edge, wg, zchunk, a, (int)ntiles, st)))
         return fail(CNV_ERR_UNSUPPORTED, "two-step tile shape not available for this block edge and dtype");
     CNV_HIP(hipGetLastError());
     if (nparts)

@@ -235,9 +235,11 @@ int cnv_diffusion_step_noalloc(const cnv_grid_desc *desc, const void *u, void *u
  * BC lists as u.  If norms is non-NULL (device array of nsteps doubles)
  * norms[k] is the FP64 sum of squares after step k; the reductions of a
  * launch run inside the next launch (one finalize launch at the end).  On
- * periodic grids (no BC list) of 16^3 or 32^3 blocks, steps go two per launch
- * (one HBM read and write for two steps) up to a multiple of four.  The loop
- * of the reference's time stepping over Field.h:457-512 / FieldOperator.h. */
+ * grids of 16^3 or 32^3 blocks that are periodic (no BC list) or whose BC
+ * lists give each domain face one rule on all its blocks (periodic on both
+ * sides of an axis, or per side Dirichlet, Symmetry of nonzero sign or
+ * Absorbing), steps go two per launch (one HBM read and write for two steps)
+ * up to a multiple of four.  The loop of the reference's time stepping over Field.h:457-512 / FieldOperator.h. */
 int cnv_diffusion_run(cnv_grid u, cnv_grid tmp, int nsteps, double nu_dt, double *norms, cnv_stream s);
 
 /* Fifth-order WENO face states (Jiang & Shu, J. Comput. Phys. 126:202-228,

@@ -125,3 +125,42 @@ def test_weno5_columns(gpu, dtype, shape, lists):
             else:
                 assert np.max(np.abs(got - ref)) <= 1e-5 * np.max(np.abs(slab))
                 assert np.linalg.norm(got - ref) <= 1e-6 * np.linalg.norm(ref)
+
+
+WALLS = {
+    "dirichlet": [(2, d, s, 0.5 - 0.25 * d + 0.125 * s) for d in range(3) for s in (0, 1)],
+    "mirror": [(3, d, s, (1.0, -1.0, 0.5)[d]) for d in range(3) for s in (0, 1)],
+    "edge": [(1, d, s, 0.0) for d in range(3) for s in (0, 1)],
+    "mixed": MIXED,
+    "z only": PARTLY,
+    "x only": [(3, 0, 0, -1.0), (2, 0, 1, 0.3)],
+    "y only": [(1, 1, 0, 0.0), (3, 1, 1, 2.0)],
+}
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("nb,edge,walls", [(nb, e, w) for w in sorted(WALLS) for nb, e in
+                                           [((1, 1, 1), 16), ((2, 3, 2), 16), ((9, 8, 7), 16), ((1, 1, 1), 32),
+                                            ((2, 1, 3), 32), ((6, 5, 3), 32)]] + [((12, 11, 13), 16, "mixed")])
+def test_run_between_walls(gpu, dtype, nb, edge, walls):
+    """Two steps per launch on grids with walls, at every z chunk the grid size
+    picks: the fields of single steps bit for bit, norms to 1e-13 (another
+    summation order)."""
+    n = (edge,) * 3
+    lists = [WALLS[walls], [], PARTLY] if nb == (2, 3, 2) else [WALLS[walls]]
+    u, slabs, _ = build(nb, n, dtype, 41, lists)
+    v, _, _ = build(nb, n, dtype, 41, lists)
+    t, _, _ = build(nb, n, dtype, 41, lists)
+    w, _, _ = build(nb, n, dtype, 41, lists)
+    dt = 0.1 / (edge * max(nb)) ** 2
+    norms, want = cnv.DeviceBuffer(8 * 7), cnv.DeviceBuffer(8 * 7)
+    res = cnv.diffusion_run(u, t, 7, dt, norms)
+    assert res is t
+    a, b = v, w
+    for k in range(7):
+        cnv.diffusion_step(a, b, dt, sumsq=want.at(8 * k))
+        a, b = b, a
+    for c in range(len(lists)):
+        assert_same(res.download(c), a.download(c), "component %d" % c)
+    gn, wn = norms.download(np.float64, 7), want.download(np.float64, 7)
+    assert np.max(np.abs(gn - wn) / wn) <= 1e-13

@@ -85,9 +85,8 @@ struct Walk3 {
 // One item of any block shape: its cells plus the face halo its operator
 // reads staged in LDS (every ghost by the lab rules), then the operator.
 template <int WG>
-__device__ __attribute__((always_inline)) inline void gen_item(const BGrid *__restrict__ grids, const BItem I, float *lds)
+__device__ __attribute__((always_inline)) inline void gen_item(const BGrid *__restrict__ grids, const BItem I, float *lds, int tid = threadIdx.x)
 {
-    const int tid = threadIdx.x;
     const BGrid &Gd = grids[I.grid];
     const int c = I.comp;
     const int nx = Gd.G.n[0], ny = Gd.G.n[1], nzb = Gd.G.n[2];
@@ -182,7 +181,7 @@ __global__ __launch_bounds__(WG) void k_batch(const BGrid *__restrict__ grids, c
 // The 7-point Euler tile body of one item on cubic blocks of edge NX (the
 // single-grid tile), run by WG threads or by one WG-thread slice (SUB).
 template <int NX, int WG, int SUB = 0>
-__device__ __attribute__((always_inline)) inline void s7_item(const BGrid *__restrict__ grids, const BItem I, float *lds)
+__device__ __attribute__((always_inline)) inline void s7_item(const BGrid *__restrict__ grids, const BItem I, float *lds, int thread = threadIdx.x)
 {
     const BGrid &Gd = grids[I.grid];
     const int c = I.comp;
@@ -192,12 +191,12 @@ __device__ __attribute__((always_inline)) inline void s7_item(const BGrid *__res
     FaceSrc<float> F[6];
     block_faces<float>(Gd.G, Gd.heads[c], Gd.has_bc[c], I.blk, cbase, F);
     (void)s7_march<float, NX, NX, WG, 1, false, SUB>(ub, ob + (long long)c * Gd.ocstride, nullptr, F, NX, I.z0,
-                                                      I.z0 + I.nz, Gd.ih2[0], Gd.ih2[1], Gd.ih2[2], Gd.nudt, lds);
+                                                      I.z0 + I.nz, Gd.ih2[0], Gd.ih2[1], Gd.ih2[2], Gd.nudt, lds, thread);
 }
 
 // The WENO5 tile body of one item on cubic blocks of edge NX.
 template <int NX, int WG, int SUB = 0>
-__device__ __attribute__((always_inline)) inline void w5_item(const BGrid *__restrict__ grids, const BItem I, float *lds)
+__device__ __attribute__((always_inline)) inline void w5_item(const BGrid *__restrict__ grids, const BItem I, float *lds, int thread = threadIdx.x)
 {
     const BGrid &Gd = grids[I.grid];
     const int c = I.comp;
@@ -207,7 +206,7 @@ __device__ __attribute__((always_inline)) inline void w5_item(const BGrid *__res
     FaceL<float> F[6];
     make_faces<float>(Gd.G, Gd.heads[c], Gd.has_bc[c], I.blk, cbase, F);
     w5_march<float, NX, NX, WG, SUB>(ub, ob + (long long)(6 * c) * Gd.ocstride, Gd.ocstride, F, NX, I.z0,
-                                     I.z0 + I.nz, lds);
+                                     I.z0 + I.nz, lds, thread);
 }
 
 // A unit of the single persistent launch.
@@ -240,7 +239,7 @@ struct OneLds {
 // the unit's items repeat its last item, writing the same values again), so
 // the tile bodies' barriers match.
 template <int WG>
-__global__ __launch_bounds__(WG) void k_batch_one(const BGrid *__restrict__ grids, const BItem *__restrict__ items,
+__global__ __launch_bounds__(WG, WG == 256 ? 4 : 3) void k_batch_one(const BGrid *__restrict__ grids, const BItem *__restrict__ items,
                                                   const BUnit *__restrict__ units, int nunits)
 {
     extern __shared__ __align__(16) float lds[];
@@ -250,21 +249,27 @@ __global__ __launch_bounds__(WG) void k_batch_one(const BGrid *__restrict__ grid
         if (u >= nunits)
             break;
         const BUnit U = units[u];
+        // the thread index is opaque per unit: as a loop invariant, the index
+        // arithmetic of all bodies was hoisted out of the loop and held in
+        // registers through every unit (151 VGPRs, three waves per SIMD; now
+        // 128 and four: 96 grids 785 -> 719 us)
+        int thread = threadIdx.x;
+        asm volatile("" : "+v"(thread));
         if (U.kind == BK_GEN) {
-            gen_item<WG>(grids, items[U.item0], lds);
+            gen_item<WG>(grids, items[U.item0], lds, thread);
         } else if (U.kind == BK_S7_32) {
-            s7_item<32, WG>(grids, items[U.item0], lds);
+            s7_item<32, WG>(grids, items[U.item0], lds, thread);
         } else if (U.kind == BK_W5_32) {
-            w5_item<32, WG>(grids, items[U.item0], lds);
+            w5_item<32, WG>(grids, items[U.item0], lds, thread);
         } else {
             // the slice index is uniform in a wave: scalar loads of the
             // item and its grid descriptor
-            const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
+            const int w = __builtin_amdgcn_readfirstlane(thread / 64);
             const BItem I = items[U.item0 + (w < U.n ? w : U.n - 1)];
             if (U.kind == BK_S7_16)
-                s7_item<16, 64, 64>(grids, I, lds + w * OneLds<WG>::S16);
+                s7_item<16, 64, 64>(grids, I, lds + w * OneLds<WG>::S16, thread);
             else
-                w5_item<16, 64, 64>(grids, I, lds + w * OneLds<WG>::W16);
+                w5_item<16, 64, 64>(grids, I, lds + w * OneLds<WG>::W16, thread);
         }
         __syncthreads(); // the next unit overwrites the tiles
     }
@@ -340,6 +345,7 @@ struct cnv_batch_s {
     // width), workgroup size
     bool one = true;
     int one_wg = 256;
+    bool one_deep = false; // many WENO5 blocks: deeper items (one_zdepth)
     std::map<std::pair<int, int>, int> zmap;
     std::vector<BItem> one_items;
     std::vector<BUnit> units;
@@ -618,13 +624,22 @@ static int launch_generic(cnv_batch_s *b, hipStream_t st)
     return CNV_OK;
 }
 
-// planes per item of the single launch for a grid (per block edge and ghost
-// width; the single-grid kernels' depths by default)
+// Planes per item of the single launch for a grid: the tuned depth of its
+// (block edge, ghost width), else by its operator.  A WENO5 item marches its
+// planes at about 2 us each, so a 32-plane item is 75 us of one workgroup: the
+// launch's tail, and all of a small batch.  WENO5 takes 8 planes (16 when the
+// batch holds 1024 32^3 blocks of it: the four extra planes a chunk reads then
+// cost more than the tail), diffusion whole blocks, other shapes 8 planes.  Us
+// per step with 32 / 16 / 8 WENO5 planes: 96 grids (2333 32^3 blocks of WENO5)
+// 716 / 683 / 693, 35 grids (354 blocks) 187 / 150 / 129, 35 small grids 78 / 43 /
+// 31; diffusion items of 8 planes instead of 32: 129 -> 140 and no gain elsewhere.
 static int one_zdepth(const cnv_batch_s *b, const cnv_batch_item &it)
 {
     const cnv_grid_s *g = it.in;
     const std::pair<int, int> key(class_key_edge(g), it.ghost);
-    int nz = b->zmap.count(key) ? b->zmap.at(key) : (key.first >= 32 ? 32 : 8);
+    int nz = !marchable(it) ? 8 : it.op == CNV_OP_DIFFUSION ? 32 : b->one_deep ? 16 : 8;
+    if (b->zmap.count(key))
+        nz = b->zmap.at(key);
     return std::max(1, std::min(nz, g->desc.block_cells[2]));
 }
 
@@ -659,6 +674,12 @@ static int build_one(cnv_batch_s *b)
         BItem item;
     };
     std::vector<Tmp> all;
+    long long weno_cells = 0;
+    for (const auto &it : b->src)
+        if (marchable(it) && it.op == CNV_OP_WENO5)
+            weno_cells += it.in->nblocks_total * it.in->desc.ncomp * it.in->desc.block_cells[0] *
+                          it.in->desc.block_cells[1] * it.in->desc.block_cells[2];
+    b->one_deep = weno_cells >= 1024LL * 32 * 32 * 32;
     for (size_t gi = 0; gi < b->src.size(); ++gi) {
         const cnv_batch_item &it = b->src[gi];
         const cnv_grid_s *g = it.in;

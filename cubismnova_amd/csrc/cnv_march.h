@@ -42,14 +42,14 @@ struct S7Shape {
 template <typename T, int NX, int NY, int WG, int MODE, bool SUMSQ, int SUB = 0>
 __device__ inline double s7_march(const T *__restrict__ ub, T *__restrict__ ob, T *__restrict__ lb,
                                   const FaceSrc<T> F[6], int NZ, int z0, int z1, T ihx2, T ihy2, T ihz2, T nudt,
-                                  T *lds)
+                                  T *lds, int thread = threadIdx.x)
 {
     using S = S7Shape<T, NX, NY, WG>;
     constexpr int VEC = S::VEC, TX = S::TX, ROWS = S::ROWS, R = S::R, P = S::P, PLANE = S::PLANE;
     static_assert(S::valid, "tile shape");
     static_assert(SUB == 0 || SUB == WG, "a slice is one tile");
     using V = VecT<T, VEC>;
-    const int tid = SUB ? (int)(threadIdx.x % SUB) : (int)threadIdx.x;
+    const int tid = SUB ? thread % SUB : thread;
     const int tx = tid % TX, ty = tid / TX;
     const int x0 = tx * VEC;
     constexpr long long SXY = (long long)NX * NY;
@@ -317,7 +317,7 @@ struct W5Shape {
 // s7_march.
 template <typename T, int NX, int NY, int WG, int SUB = 0>
 __device__ inline void w5_march(const T *__restrict__ ub, T *__restrict__ ob, long long ocstride,
-                                const FaceL<T> F[6], int NZ, int z0, int z1, T *lds)
+                                const FaceL<T> F[6], int NZ, int z0, int z1, T *lds, int thread = threadIdx.x)
 {
     using S = W5Shape<T, NX, NY, WG>;
     constexpr int G = S::G, VEC = S::VEC, TX = S::TX, ROWS = S::ROWS, R = S::R, P = S::P, PLANE = S::PLANE;
@@ -325,7 +325,7 @@ __device__ inline void w5_march(const T *__restrict__ ub, T *__restrict__ ob, lo
     static_assert(S::valid, "tile shape");
     static_assert(SUB == 0 || SUB == WG, "a slice is one tile");
     using V = VecT<T, VEC>;
-    const int tid = SUB ? (int)(threadIdx.x % SUB) : (int)threadIdx.x;
+    const int tid = SUB ? thread % SUB : thread;
     const FaceL<T> FX0 = F[0], FX1 = F[1], FY0 = F[2], FY1 = F[3], FZ0 = F[4], FZ1 = F[5];
 
     const int tx = tid % TX, ty = tid / TX;

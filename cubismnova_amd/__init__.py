@@ -300,6 +300,7 @@ class Cartesian:
         self.nblocks_total = nb[0] * nb[1] * nb[2]
         self._mesh = _Mesh(b, e, [nb[k] * bc[k] for k in range(3)])
         self._bcs = {}
+        self._red = None
 
     @classmethod
     def from_tensor(cls, t, nblocks, block_cells, begin=0.0, end=1.0, ncomp=1, entity="cell"):
@@ -442,6 +443,13 @@ class Cartesian:
             out = DeviceBuffer(n * self.dtype.itemsize)
         call("cnv_lab_load_all", self.handle, comp, ctypes.byref(sc), out.ptr, _st(stream))
         return out, list(ext)
+
+    def _reductions(self):
+        """Device memory of this grid's reduction results, kept with the
+        partial sums the grid holds (allocated by the first reduction)."""
+        if self._red is None:
+            self._red = DeviceBuffer(24)
+        return self._red
 
     def __del__(self):
         try:
@@ -628,7 +636,7 @@ def CartesianReadHDF(fname, grid, face_dir=0, file_dtype=None):
 
 def grid_sums(g, comp=0, stream=None):
     """(sum, sum of squares) of one component, FP64, deterministic."""
-    buf = DeviceBuffer(16)
+    buf = g._reductions()
     call("cnv_grid_sums", g.handle, comp, buf.ptr, _st(stream))
     r = buf.download(np.float64, 2, stream)
     return float(r[0]), float(r[1])
@@ -820,7 +828,7 @@ def jacobi_solve(u, f, work, refine=True, sweeps_per_cycle=50, max_cycles=1000, 
 
 def grid_compare(a, b, comp_a=0, comp_b=0, stream=None):
     """(sum (a-b)^2, sum b^2, max|a-b|) over one component, FP64 on the device."""
-    buf = DeviceBuffer(24)
+    buf = a._reductions()
     call("cnv_grid_compare", a.handle, comp_a, b.handle, comp_b, buf.ptr, _st(stream))
     r = buf.download(np.float64, 3, stream)
     return float(r[0]), float(r[1]), float(r[2])

@@ -72,27 +72,93 @@ int ensure_bc_table(cnv_grid_s *g, int comp)
         resolve_faces(entries.data() + heads[(size_t)b].offset, (int)lst.size(), sb, se, heads[(size_t)b].kind,
                       heads[(size_t)b].val);
     }
-    if (t.heads || t.entries) {
+    if (t.heads) {
         // the table is rewritten (BC lists changed): kernels still queued on
         // any stream may read it, so they finish first
         CNV_HIP(hipDeviceSynchronize());
     }
-    if (!t.heads)
-        CNV_HIP(hipMalloc((void **)&t.heads, sizeof(DevBCHead) * (size_t)nb));
-    if ((int)entries.size() > t.nentries_cap) {
-        if (t.entries)
-            CNV_HIP(hipFree(t.entries));
-        t.entries = nullptr;
-        t.nentries_cap = (int)entries.size();
-        CNV_HIP(hipMalloc((void **)&t.entries, sizeof(DevBC) * (size_t)t.nentries_cap));
+    const size_t hb = sizeof(DevBCHead) * (size_t)nb, eb = sizeof(DevBC) * entries.size();
+    if (hb + eb > t.bytes_cap) {
+        if (t.heads)
+            CNV_HIP(hipFree(t.heads));
+        t.heads = nullptr;
+        t.bytes_cap = 0;
+        CNV_HIP(hipMalloc((void **)&t.heads, hb + eb));
+        t.bytes_cap = hb + eb;
     }
-    CNV_HIP(hipMemcpy(t.heads, heads.data(), sizeof(DevBCHead) * (size_t)nb, hipMemcpyHostToDevice));
-    if (!entries.empty())
-        CNV_HIP(hipMemcpy(t.entries, entries.data(), sizeof(DevBC) * entries.size(),
-                          hipMemcpyHostToDevice));
+    t.entries = reinterpret_cast<DevBC *>(reinterpret_cast<char *>(t.heads) + hb);
+    std::vector<char> image(hb + eb);
+    std::memcpy(image.data(), heads.data(), hb);
+    if (eb)
+        std::memcpy(image.data() + hb, entries.data(), eb);
+    CNV_HIP(hipMemcpy(t.heads, image.data(), hb + eb, hipMemcpyHostToDevice));
     t.any = any;
     t.version = g->bc_version;
     return CNV_OK;
+}
+
+// Every block's BC list resolved for a stencil that reads both sides (-1, 2)
+// gives the six faces (resolve_faces).  Uniform: neighbour copies on every
+// face inside the domain and, on each domain face, the same rule on every
+// block of that face: a periodic neighbour on both sides of an axis, or on
+// each side a Dirichlet constant, a Symmetry mirror of nonzero sign, or an
+// Absorbing edge copy.
+const FaceInfo &face_info(cnv_grid_s *g, int comp)
+{
+    FaceInfo &F = g->tables[comp].faces;
+    if (F.version == g->bc_version)
+        return F;
+    F = FaceInfo();
+    const int *nb = g->desc.nblocks;
+    const int sb[3] = {-1, -1, -1}, se[3] = {2, 2, 2};
+    int kind0[3][2];
+    double val0[3][2];
+    for (int d = 0; d < 3; ++d)
+        for (int s = 0; s < 2; ++s) {
+            kind0[d][s] = -1;
+            val0[d][s] = 0.0;
+        }
+    F.uniform = true;
+    std::vector<DevBC> tmp;
+    for (long long b = 0; b < g->nblocks_total; ++b) {
+        const int bi[3] = {(int)(b % nb[0]), (int)((b / nb[0]) % nb[1]), (int)(b / ((long long)nb[0] * nb[1]))};
+        const auto &l = g->bcs[comp][(size_t)b];
+        tmp.clear();
+        for (const auto &x : l)
+            tmp.push_back({x.kind, x.dir, x.side, 0, x.value});
+        F.longest = l.size() > F.longest ? l.size() : F.longest;
+        int kind[6];
+        double val[6];
+        resolve_faces(tmp.data(), (int)tmp.size(), sb, se, kind, val);
+        for (int f = 0; f < 6; ++f) {
+            const int d = f >> 1, s = f & 1;
+            F.unset = F.unset || kind[f] == FACE_UNSET;
+            if (bi[d] != (s == 0 ? 0 : nb[d] - 1)) {
+                F.uniform = F.uniform && kind[f] == FACE_NBR;
+                continue;
+            }
+            if (kind[f] == FACE_UNSET || (kind[f] == FACE_SYMMETRY && val[f] == 0.0))
+                F.uniform = false;
+            const double v = (kind[f] == FACE_DIRICHLET || kind[f] == FACE_SYMMETRY) ? val[f] : 0.0;
+            if (kind0[d][s] < 0) {
+                kind0[d][s] = kind[f];
+                val0[d][s] = v;
+            } else if (kind[f] != kind0[d][s] || v != val0[d][s]) {
+                F.uniform = false;
+            }
+        }
+    }
+    for (int d = 0; d < 3; ++d) {
+        F.uniform = F.uniform && (kind0[d][0] == FACE_NBR) == (kind0[d][1] == FACE_NBR);
+        for (int s = 0; s < 2; ++s) {
+            const int k = kind0[d][s];
+            F.fm[d][s] = k == FACE_NBR ? FM_PERIODIC : k == FACE_DIRICHLET ? FM_CONST : k == FACE_SYMMETRY ? FM_MIRROR
+                                                                                                          : FM_EDGE;
+            F.fv[d][s] = val0[d][s];
+        }
+    }
+    F.version = g->bc_version;
+    return F;
 }
 
 int ensure_partials(cnv_grid_s *g, size_t n)
@@ -387,8 +453,6 @@ int cnv_grid_destroy(cnv_grid g)
     for (auto &t : g->tables) {
         if (t.heads)
             (void)hipFree(t.heads);
-        if (t.entries)
-            (void)hipFree(t.entries);
     }
     if (g->partials)
         (void)hipFree(g->partials);
@@ -396,6 +460,8 @@ int cnv_grid_destroy(cnv_grid g)
         (void)hipFree(g->czm_dev);
     if (g->czp_dev)
         (void)hipFree(g->czp_dev);
+    if (g->solve_host)
+        (void)hipHostFree(g->solve_host);
     delete g;
     return CNV_OK;
 }
@@ -713,7 +779,7 @@ int cnv_diffusion_run(cnv_grid u, cnv_grid tmp, int nsteps, double nu_dt, double
     if (nsteps < 0)
         return fail(CNV_ERR_INVALID, "nsteps must be >= 0");
     // tmp is read as the source of every other step: same BCs as u
-    if (nsteps > 1) {
+    if (nsteps > 1 && (u->bc_version || tmp->bc_version)) {
         std::lock_guard<std::mutex> lk(tmp->mtx);
         bool same = true;
         for (int c = 0; c < u->desc.ncomp && same; ++c)
@@ -928,15 +994,24 @@ int cnv_add_correction(cnv_grid u, int cu, cnv_grid e, int ce, cnv_stream s)
 static void copy_bcs(cnv_grid_s *src, cnv_grid_s *dst, int c, bool homogeneous)
 {
     std::lock_guard<std::mutex> lk(dst->mtx);
+    bool changed = false;
     for (long long b = 0; b < dst->nblocks_total; ++b) {
         auto l = src->bcs[0][(size_t)b];
         if (homogeneous)
             for (auto &x : l)
                 if (x.kind == CNV_BC_DIRICHLET)
                     x.value = 0.0;
-        dst->bcs[c][(size_t)b] = l;
+        auto &t = dst->bcs[c][(size_t)b];
+        bool same = t.size() == l.size();
+        for (size_t i = 0; same && i < l.size(); ++i)
+            same = t[i].kind == l[i].kind && t[i].dir == l[i].dir && t[i].side == l[i].side && t[i].value == l[i].value;
+        if (!same) {
+            t = l;
+            changed = true;
+        }
     }
-    ++dst->bc_version;
+    if (changed) // an unchanged list keeps its device table
+        ++dst->bc_version;
 }
 
 int cnv_jacobi_solve(cnv_grid u, cnv_grid f, cnv_grid work, const cnv_solve_opts *o, cnv_solve_info *info,
@@ -968,8 +1043,8 @@ int cnv_jacobi_solve(cnv_grid u, cnv_grid f, cnv_grid work, const cnv_solve_opts
     copy_bcs(u, work, 0, refine);
     if (refine)
         copy_bcs(u, work, 1, true);
-    // set up metric and BC tables now: nothing may allocate inside the capture
     CNV_CHECK(jacobi_prepare(u, 0));
+    hipStream_t st = (hipStream_t)s;
     {
         std::lock_guard<std::mutex> lk(work->mtx);
         const int nz = u->desc.nblocks[2] * u->desc.block_cells[2];
@@ -977,113 +1052,81 @@ int cnv_jacobi_solve(cnv_grid u, cnv_grid f, cnv_grid work, const cnv_solve_opts
             CNV_HIP(hipMalloc((void **)&work->czm_dev, sizeof(double) * nz));
             CNV_HIP(hipMalloc((void **)&work->czp_dev, sizeof(double) * nz));
         }
-        CNV_HIP(hipMemcpy(work->czm_dev, u->czm_dev, sizeof(double) * nz, hipMemcpyDeviceToDevice));
-        CNV_HIP(hipMemcpy(work->czp_dev, u->czp_dev, sizeof(double) * nz, hipMemcpyDeviceToDevice));
+        CNV_HIP(hipMemcpyAsync(work->czm_dev, u->czm_dev, sizeof(double) * nz, hipMemcpyDeviceToDevice, st));
+        CNV_HIP(hipMemcpyAsync(work->czp_dev, u->czp_dev, sizeof(double) * nz, hipMemcpyDeviceToDevice, st));
+        if (!work->solve_host)
+            CNV_HIP(hipHostMalloc((void **)&work->solve_host, 4 * sizeof(double), hipHostMallocDefault));
     }
     CNV_CHECK(jacobi_prepare(work, 0));
     CNV_CHECK(jacobi_prepare(work, 1));
-    hipStream_t st = (hipStream_t)s;
-    hipStream_t cs;
-    CNV_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
-    double *dev = nullptr; // [0] = |f|^2 pieces, [2] = |r|^2
+    // The reductions write |f|^2 and |r|^2 into pinned host memory: the host
+    // reads them after it waited for the stream, with no copy in between.
+    // The launches of a cycle go straight to the caller's stream: recording
+    // and instantiating a graph per call took longer (about 0.3 ms) than a
+    // replay saves over the calls of a solve (0.4 us per launch).
+    double *hst = work->solve_host; // [0] sum f, [1] sum f^2, [2] sum r^2
     int rc = CNV_OK;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    double hst[3] = {0, 0, 0};
     const int S = o->sweeps_per_cycle;
     long long sweeps = 0;
     int cycles = 0;
     double rel = 0.0;
-    auto defect = [&](hipStream_t q) -> int {
+    auto defect = [&]() -> int {
         // refine: r (FP32, work comp 2) = f - A u in FP64; plain: work comp 1
-        return launch_jacobi(u, 0, f, 0, work, refine ? 2 : 1, 1, 0.0, dev + 2, q);
+        return launch_jacobi(u, 0, f, 0, work, refine ? 2 : 1, 1, 0.0, hst + 2, st);
     };
-    do {
-        if (hipMalloc((void **)&dev, 3 * sizeof(double)) != hipSuccess) {
-            rc = fail(CNV_ERR_ALLOC, "solver scratch");
-            break;
-        }
-        if (st)
-            CNV_HIP(hipStreamSynchronize(st));
-        rc = launch_sums(f, 0, dev, cs);
-        if (rc != CNV_OK)
-            break;
-        rc = defect(cs);
-        if (rc != CNV_OK)
-            break;
-        CNV_HIP(hipMemcpyAsync(hst, dev, 3 * sizeof(double), hipMemcpyDeviceToHost, cs));
-        CNV_HIP(hipStreamSynchronize(cs));
-        const double fn = std::sqrt(hst[1]);
-        if (!(fn > 0.0)) {
-            rel = 0.0;
-            break;
-        }
-        rel = std::sqrt(hst[2]) / fn;
-        if (history && history_cap > 0)
-            history[0] = rel;
-        // one cycle, recorded once and replayed (relaxed capture: see
-        // cnv_graph_begin)
-        CNV_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeRelaxed));
-        // sweep pairs in one launch each where the faces allow it (the same
-        // values as single sweeps, u and f read once per pair)
+    // sweep pairs in one launch each where the faces allow it (the same
+    // values as single sweeps, u and f read once per pair)
+    const bool two = refine ? jacobi2_applies(work, 0, work, work) && jacobi2_applies(work, 1, work, work)
+                            : jacobi2_applies(u, 0, f, work) && jacobi2_applies(work, 0, f, u);
+    auto cycle = [&]() -> int {
         int crc = CNV_OK;
         if (refine) {
-            const bool two = jacobi2_applies(work, 0, work, work) && jacobi2_applies(work, 1, work, work);
-            crc = launch_fill((char *)work->data, CNV_F32, 0.0, work->component_bytes / 4, cs);
+            crc = launch_fill((char *)work->data, CNV_F32, 0.0, work->component_bytes / 4, st);
             const int L = two ? S / 2 : S;
             for (int k = 0; k < L && crc == CNV_OK; ++k)
-                crc = two ? launch_jacobi2(work, k % 2, work, 2, work, 1 - k % 2, o->omega, cs, nullptr)
-                          : launch_jacobi(work, k % 2, work, 2, work, 1 - k % 2, 0, o->omega, nullptr, cs);
+                crc = two ? launch_jacobi2(work, k % 2, work, 2, work, 1 - k % 2, o->omega, st, nullptr)
+                          : launch_jacobi(work, k % 2, work, 2, work, 1 - k % 2, 0, o->omega, nullptr, st);
             if (crc == CNV_OK)
-                crc = launch_correct(u, 0, work, L % 2, cs);
+                crc = launch_correct(u, 0, work, L % 2, st);
         } else {
             // an even number of pair launches (u -> work -> u ...), then the
             // remaining two sweeps, if any, one at a time: the cycle ends in u
-            const bool two = jacobi2_applies(u, 0, f, work) && jacobi2_applies(work, 0, f, u);
             const int pairs = two ? (S / 2) & ~1 : 0;
             for (int k = 0; k < pairs + (S - 2 * pairs) && crc == CNV_OK; ++k) {
                 cnv_grid_s *a = k % 2 == 0 ? u : work, *b = k % 2 == 0 ? work : u;
-                crc = k < pairs ? launch_jacobi2(a, 0, f, 0, b, 0, o->omega, cs, nullptr)
-                                : launch_jacobi(a, 0, f, 0, b, 0, 0, o->omega, nullptr, cs);
+                crc = k < pairs ? launch_jacobi2(a, 0, f, 0, b, 0, o->omega, st, nullptr)
+                                : launch_jacobi(a, 0, f, 0, b, 0, 0, o->omega, nullptr, st);
             }
         }
-        if (crc == CNV_OK)
-            crc = defect(cs);
-        hipError_t ce = hipStreamEndCapture(cs, &graph);
-        if (crc != CNV_OK) {
-            rc = crc;
-            break;
-        }
-        if (ce != hipSuccess) {
-            rc = hip_fail(ce, "hipStreamEndCapture");
-            break;
-        }
-        if (hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) != hipSuccess) {
-            rc = fail(CNV_ERR_HIP, "hipGraphInstantiate failed");
-            break;
-        }
-        while (cycles < o->max_cycles && rel > o->tol) {
-            CNV_HIP(hipGraphLaunch(exec, cs));
-            CNV_HIP(hipMemcpyAsync(hst + 2, dev + 2, sizeof(double), hipMemcpyDeviceToHost, cs));
-            CNV_HIP(hipStreamSynchronize(cs));
-            ++cycles;
-            sweeps += S;
+        return crc == CNV_OK ? defect() : crc;
+    };
+    rc = launch_sums(f, 0, hst, st);
+    if (rc == CNV_OK)
+        rc = defect();
+    if (rc == CNV_OK) {
+        CNV_HIP(hipStreamSynchronize(st));
+        const double fn = std::sqrt(hst[1]);
+        if (fn > 0.0) {
             rel = std::sqrt(hst[2]) / fn;
-            if (history && cycles < history_cap)
-                history[cycles] = rel;
-            if (!std::isfinite(rel)) {
-                rc = fail(CNV_ERR_INVALID, "solver diverged (non-finite residual)");
-                break;
+            if (history && history_cap > 0)
+                history[0] = rel;
+            while (cycles < o->max_cycles && rel > o->tol) {
+                rc = cycle();
+                if (rc != CNV_OK)
+                    break;
+                CNV_HIP(hipStreamSynchronize(st));
+                ++cycles;
+                sweeps += S;
+                rel = std::sqrt(hst[2]) / fn;
+                if (history && cycles < history_cap)
+                    history[cycles] = rel;
+                if (!std::isfinite(rel)) {
+                    rc = fail(CNV_ERR_INVALID, "solver diverged (non-finite residual)");
+                    break;
+                }
             }
         }
-    } while (false);
-    if (exec)
-        (void)hipGraphExecDestroy(exec);
-    if (graph)
-        (void)hipGraphDestroy(graph);
-    if (dev)
-        (void)hipFree(dev);
-    (void)hipStreamDestroy(cs);
+    }
     info->cycles = cycles;
     info->sweeps = sweeps;
     info->rel_residual = rel;

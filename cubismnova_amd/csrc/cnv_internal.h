@@ -61,11 +61,33 @@ struct Geom {
 
 // ------------------------------------------------------------ host grid object
 
+// Rule of a domain face as the two-step and two-sweep kernels apply it to the
+// ghost cells they read past it: the periodic neighbour, a constant
+// (Dirichlet, BC/Dirichlet.h:75-113), sign times the mirror cell (Symmetry,
+// BC/Symmetry.h:69-114: ghost layer l reads interior cell l - 1 from the
+// face), or the face's own cell (Absorbing, BC/Absorbing.h:66-105: every
+// layer reads interior cell 0 from the face).
+enum { FM_PERIODIC = 0, FM_CONST = 1, FM_MIRROR = 2, FM_EDGE = 3 };
+
+// What the BC lists of one component say about the faces of its blocks
+// (host side, for the stencils that read ghosts on both sides).
+struct FaceInfo {
+    uint64_t version = ~0ull; // BC version this was derived from
+    bool unset = false;       // some face has ghosts that no rule writes
+    size_t longest = 0;       // entries of the longest list
+    // every domain face has one rule (FM_*) on all its blocks and every inner
+    // face is a neighbour copy: the rules and their constants or signs
+    bool uniform = false;
+    int fm[3][2] = {};
+    double fv[3][2] = {};
+};
+
 struct BCTable {
+    FaceInfo faces;
     uint64_t version = ~0ull; // BC version this table was built from
-    DevBCHead *heads = nullptr;
+    DevBCHead *heads = nullptr; // one allocation: the heads, then the entries
     DevBC *entries = nullptr;
-    int nentries_cap = 0;
+    size_t bytes_cap = 0;
     bool any = false; // false: no block of this component carries a BC
 };
 
@@ -95,6 +117,10 @@ struct cnv_grid_s {
     double *czm_dev = nullptr;
     double *czp_dev = nullptr;
     size_t partials_cap = 0;
+
+    // pinned host memory (4 doubles) that the solver's reductions write,
+    // allocated by the first solve that uses this grid as its work grid
+    double *solve_host = nullptr;
 
     std::mutex mtx;
 };
@@ -147,23 +173,30 @@ inline cnv::Geom geom_of(const cnv_grid_s *g)
 int grid_layout(const cnv_grid_desc *desc, cnv_grid_s *g);
 // Upload (if stale) the BC table of component comp; returns status.
 int ensure_bc_table(cnv_grid_s *g, int comp);
+// The faces of component comp, derived again when its BC lists changed; the
+// caller holds the grid's mutex.
+const FaceInfo &face_info(cnv_grid_s *g, int comp);
 // Make sure the reduction scratch holds at least n partials.
 int ensure_partials(cnv_grid_s *g, size_t n);
 
 int check_stencil(const cnv_stencil *s);
 
 // Resolve one block's ordered BC list into six faces for a non-tensorial
-// stencil; shared by host and device.  Rule (FieldLab.h:206-223 with the
-// BC slabs of BC/*.h): the face (dir, side) starts as a neighbour copy unless
-// the last BC of `dir` is non-periodic with that side (then unwritten); every
-// non-Base BC on that face whose stencil has width in `dir`
-// (BC/Base.h:73-78) overwrites the whole slab, so the last one decides.
-// Loops run over compile-time face indices so that device code keeps the
-// arrays in registers.
-__host__ __device__ inline void resolve_faces(const DevBC *list, int n, const int sb[3],
-                                              const int se[3], int kind[6], double value[6])
+// stencil (host side: the kernels read the result from the BC table).  Rule
+// (FieldLab.h:206-223 with the BC slabs of BC/*.h): the face (dir, side)
+// starts as a neighbour copy unless the last BC of `dir` is non-periodic with
+// that side (then unwritten); every non-Base BC on that face whose stencil has
+// width in `dir` (BC/Base.h:73-78) overwrites the whole slab, so the last one
+// decides.
+inline void resolve_faces(const DevBC *list, int n, const int sb[3], const int se[3], int kind[6], double value[6])
 {
-#pragma unroll
+    if (n == 0) { // no list: six neighbour copies
+        for (int f = 0; f < 6; ++f) {
+            kind[f] = FACE_NBR;
+            value[f] = 0.0;
+        }
+        return;
+    }
     for (int f = 0; f < 6; ++f) {
         const int dir = f >> 1, side = f & 1;
         bool periodic = true;
@@ -216,13 +249,6 @@ int launch_diffusion_noalloc(const cnv_grid_desc *desc, const void *u, void *u_n
 
 int launch_sums(cnv_grid_s *g, int comp, double *out, hipStream_t st);
 int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_dt, double *norms, hipStream_t st);
-// Rule of a domain face as the two-step and two-sweep kernels apply it to the
-// ghost cells they read past it: the periodic neighbour, a constant
-// (Dirichlet, BC/Dirichlet.h:75-113), sign times the mirror cell (Symmetry,
-// BC/Symmetry.h:69-114: ghost layer l reads interior cell l - 1 from the
-// face), or the face's own cell (Absorbing, BC/Absorbing.h:66-105: every
-// layer reads interior cell 0 from the face).
-enum { FM_PERIODIC = 0, FM_CONST = 1, FM_MIRROR = 2, FM_EDGE = 3 };
 // the six rules of a component; false unless every domain face has one rule on
 // all its blocks and every inner face is a neighbour copy (cnv_jacobi2.hip)
 bool jacobi2_faces(cnv_grid_s *g, int comp, int fm[3][2], double fv[3][2]);

@@ -482,20 +482,8 @@ int launch_jacobi(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out,
         rc = ensure_bc_table(u, cu);
         if (rc != CNV_OK)
             return rc;
-        const int sb[3] = {-1, -1, -1}, se[3] = {2, 2, 2};
-        for (const auto &l : u->bcs[cu]) {
-            if (l.empty())
-                continue;
-            std::vector<DevBC> tmp;
-            for (const auto &b : l)
-                tmp.push_back({b.kind, b.dir, b.side, 0, b.value});
-            int kind[6];
-            double val[6];
-            resolve_faces(tmp.data(), (int)tmp.size(), sb, se, kind, val);
-            for (int k = 0; k < 6; ++k)
-                if (kind[k] == FACE_UNSET)
-                    return fail(CNV_ERR_UNSUPPORTED, "BC list leaves ghost cells unwritten");
-        }
+        if (face_info(u, cu).unset)
+            return fail(CNV_ERR_UNSUPPORTED, "BC list leaves ghost cells unwritten");
         const BCTable &t = u->tables[cu];
         a.has_bc = (t.any && t.heads) ? 1 : 0;
         a.heads = t.heads;

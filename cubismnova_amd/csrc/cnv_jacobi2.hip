@@ -794,70 +794,20 @@ int jacobi2_get_tune(int dtype, int edge, int *wg, int *zchunk, int *split)
     return CNV_OK;
 }
 
-// The grid's domain faces as the two-sweep kernel needs them (component
-// comp): every block's BC list resolved for the sweep's stencil (-1, 2)
-// gives neighbour copies on every face inside the domain and, on each domain
-// face, the same rule on every block of that face: a periodic neighbour on
-// both sides of an axis, or on each side a Dirichlet constant, a Symmetry
-// mirror of nonzero sign, or an Absorbing edge copy.  Fills fm and fv;
-// false otherwise.
+// The rules of a component's domain faces as the two-sweep kernel needs them.
 bool jacobi2_faces(cnv_grid_s *g, int comp, int fm[3][2], double fv[3][2])
 {
-    const int *nb = g->desc.nblocks;
     std::lock_guard<std::mutex> lk(g->mtx);
-    const auto &lists = g->bcs[comp];
-    const int sb[3] = {-1, -1, -1}, se[3] = {2, 2, 2};
-    int kind0[3][2];
-    double val0[3][2];
+    const FaceInfo &f = face_info(g, comp);
     for (int d = 0; d < 3; ++d)
-        for (int s = 0; s < 2; ++s) {
-            kind0[d][s] = -1;
-            val0[d][s] = 0.0;
+        for (int k = 0; k < 2; ++k) {
+            fm[d][k] = f.fm[d][k];
+            fv[d][k] = f.fv[d][k];
         }
-    for (long long b = 0; b < g->nblocks_total; ++b) {
-        const int bi[3] = {(int)(b % nb[0]), (int)((b / nb[0]) % nb[1]), (int)(b / ((long long)nb[0] * nb[1]))};
-        std::vector<DevBC> tmp;
-        for (const auto &x : lists[(size_t)b])
-            tmp.push_back({x.kind, x.dir, x.side, 0, x.value});
-        int kind[6];
-        double val[6];
-        resolve_faces(tmp.data(), (int)tmp.size(), sb, se, kind, val);
-        for (int f = 0; f < 6; ++f) {
-            const int d = f >> 1, s = f & 1;
-            const bool edge = bi[d] == (s == 0 ? 0 : nb[d] - 1);
-            if (!edge) {
-                if (kind[f] != FACE_NBR)
-                    return false;
-                continue;
-            }
-            if (kind[f] == FACE_UNSET || (kind[f] == FACE_SYMMETRY && val[f] == 0.0))
-                return false;
-            const double v = (kind[f] == FACE_DIRICHLET || kind[f] == FACE_SYMMETRY) ? val[f] : 0.0;
-            if (kind0[d][s] < 0) {
-                kind0[d][s] = kind[f];
-                val0[d][s] = v;
-            } else if (kind[f] != kind0[d][s] || v != val0[d][s]) {
-                return false;
-            }
-        }
-    }
-    for (int d = 0; d < 3; ++d) {
-        const bool p0 = kind0[d][0] == FACE_NBR, p1 = kind0[d][1] == FACE_NBR;
-        if (p0 != p1)
-            return false;
-        for (int s = 0; s < 2; ++s) {
-            const int k = kind0[d][s];
-            fm[d][s] = k == FACE_NBR ? FM_PERIODIC : k == FACE_DIRICHLET ? FM_CONST : k == FACE_SYMMETRY ? FM_MIRROR
-                                                                                                        : FM_EDGE;
-            fv[d][s] = val0[d][s];
-        }
-    }
     // a periodic or mirror z reads planes two cells past the grid from
     // inside it with one addition
-    const int ngz = nb[2] * g->desc.block_cells[2];
-    if (ngz < 2 && (fm[2][0] == FM_PERIODIC || fm[2][0] == FM_MIRROR || fm[2][1] == FM_MIRROR))
-        return false;
-    return true;
+    const int ngz = g->desc.nblocks[2] * g->desc.block_cells[2];
+    return f.uniform && !(ngz < 2 && (fm[2][0] == FM_PERIODIC || fm[2][0] == FM_MIRROR || fm[2][1] == FM_MIRROR));
 }
 
 // Whether the two-sweep kernel runs u -> out on these grids (u, f, out of

@@ -438,26 +438,15 @@ static bool force_generic()
     return g_force_generic == 1;
 }
 
-// Host check that every face the operator reads is written by the lab rules.
+// Host check that every face the operator reads is written by the lab rules
+// (the caller holds the grid's mutex).
 static int check_faces(cnv_grid_s *g, int comp)
 {
-    const int sb[3] = {-1, -1, -1}, se[3] = {2, 2, 2};
-    DevBC tmp[64];
-    for (const auto &l : g->bcs[comp]) {
-        if (l.empty())
-            continue;
-        if (l.size() > 64)
-            return fail(CNV_ERR_UNSUPPORTED, "BC list too long");
-        for (size_t k = 0; k < l.size(); ++k)
-            tmp[k] = {l[k].kind, l[k].dir, l[k].side, 0, l[k].value};
-        int kind[6];
-        double val[6];
-        resolve_faces(tmp, (int)l.size(), sb, se, kind, val);
-        for (int f = 0; f < 6; ++f)
-            if (kind[f] == FACE_UNSET)
-                return fail(CNV_ERR_UNSUPPORTED,
-                            "BC list leaves ghost cells of a face unwritten for Stencil(-1,2)");
-    }
+    const FaceInfo &f = face_info(g, comp);
+    if (f.longest > 64)
+        return fail(CNV_ERR_UNSUPPORTED, "BC list too long");
+    if (f.unset)
+        return fail(CNV_ERR_UNSUPPORTED, "BC list leaves ghost cells of a face unwritten for Stencil(-1,2)");
     return CNV_OK;
 }
 

@@ -670,9 +670,8 @@ bool x2_applicable(cnv_grid_s *u)
         return false;
     std::lock_guard<std::mutex> lk(u->mtx);
     for (int c = 0; c < u->desc.ncomp; ++c)
-        for (const auto &l : u->bcs[c])
-            if (!l.empty())
-                return false;
+        if (face_info(u, c).longest > 0)
+            return false;
     return true;
 }
 

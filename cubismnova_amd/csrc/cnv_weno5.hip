@@ -328,26 +328,6 @@ static int w5_run(W5Args &a, hipStream_t st, const W5Tune *over)
     return w5_cols<T>(a, st);
 }
 
-static int check_faces_w5(cnv_grid_s *g, int comp)
-{
-    const int sb[3] = {-3, -3, -3}, se[3] = {4, 4, 4};
-    std::vector<DevBC> tmp;
-    for (const auto &l : g->bcs[comp]) {
-        if (l.empty())
-            continue;
-        tmp.clear();
-        for (const auto &b : l)
-            tmp.push_back({b.kind, b.dir, b.side, 0, b.value});
-        int kind[6];
-        double val[6];
-        resolve_faces(tmp.data(), (int)tmp.size(), sb, se, kind, val);
-        for (int f = 0; f < 6; ++f)
-            if (kind[f] == FACE_UNSET)
-                return fail(CNV_ERR_UNSUPPORTED, "BC list leaves ghost cells of a face unwritten for Stencil(-3,4)");
-    }
-    return CNV_OK;
-}
-
 int launch_weno5(cnv_grid_s *in, cnv_grid_s *out, hipStream_t st, const int *tile)
 {
     const int nc = in->desc.ncomp;
@@ -368,9 +348,9 @@ int launch_weno5(cnv_grid_s *in, cnv_grid_s *out, hipStream_t st, const int *til
             int rc = ensure_bc_table(in, c);
             if (rc != CNV_OK)
                 return rc;
-            rc = check_faces_w5(in, c);
-            if (rc != CNV_OK)
-                return rc;
+            if (face_info(in, c).unset)
+                return fail(CNV_ERR_UNSUPPORTED,
+                            "BC list leaves ghost cells of a face unwritten for Stencil(-3,4)");
             a.has_bc[c] = (in->tables[c].any && in->tables[c].heads) ? 1 : 0;
             a.heads[c] = in->tables[c].heads;
         }

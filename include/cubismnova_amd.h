@@ -332,8 +332,8 @@ typedef struct {
  * FP32 defect); each cycle zeroes e, runs sweeps_per_cycle FP32 sweeps on
  * A e = r with u's BCs made homogeneous, adds e to u in FP64 and recomputes
  * the FP64 defect.  refine = 0: plain sweeps in u's dtype, work of u's dtype
- * with 2 components.  One cycle is recorded once into a HIP graph and
- * replayed; the relative residual after cycle c goes to history[c]
+ * with 2 components.  The launches go to stream s, which the host waits for
+ * once per cycle; the relative residual after cycle c goes to history[c]
  * (history[0] = initial).  Calls on the same grids must not overlap. */
 int cnv_jacobi_solve(cnv_grid u, cnv_grid f, cnv_grid work, const cnv_solve_opts *opts, cnv_solve_info *info,
                      double *history, int history_cap, cnv_stream s);

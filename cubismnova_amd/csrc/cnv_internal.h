@@ -233,6 +233,7 @@ int launch_lab(const cnv_grid_s *g, int comp, const cnv_stencil &s, bool apply_b
 int ensure_zmetric(cnv_grid_s *g);
 // two Jacobi sweeps per launch on grids whose axes are periodic or carry one
 // Dirichlet constant per domain face (cnv_jacobi2.hip)
+int jacobi2_tile_sweeps(const cnv_grid_s *u);
 bool jacobi2_applies(cnv_grid_s *u, int cu, cnv_grid_s *f, cnv_grid_s *out);
 int launch_jacobi2(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out, int co, double omega,
                    hipStream_t st, const int *tile);
@@ -261,13 +262,25 @@ struct X2Faces {
     double fv[3][2];
 };
 
-bool x2_walls(cnv_grid_s *u, X2Faces *faces);
+bool run_walls(cnv_grid_s *u, X2Faces *faces);
+bool run_periodic(cnv_grid_s *u);
+bool x2_shape_ok(const cnv_grid_s *u);
 bool x2_applicable(cnv_grid_s *u);
 long long x2_tiles(const cnv_grid_s *u, int zchunk);
-void x2_tile(cnv_grid_s *u, int *wg, int *zchunk);
+bool x2_tile(cnv_grid_s *u, int *wg, int *zchunk);
 int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *part1, double *part2,
                         const double *const prev_p[2], const int prev_n[2], double *const prev_out[2], int wg,
                         int zchunk, int *nparts, hipStream_t st, const X2Faces *faces = nullptr);
+// 2 or 4 Euler steps or Jacobi sweeps per launch on LDS tiles of the domain, any
+// block shape (cnv_tile.hip): tiles of a launch, the steps a grid takes (0:
+// another kernel), the launches; the launches of n steps, up to k at a time
+int tile_count(const cnv_grid_s *u, int k, int ncomp);
+int tile_steps(const cnv_grid_s *u, bool marching);
+int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int k, double nu_dt, double *part, const double *prev_p,
+                      int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st);
+int launch_tile_jacobi(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out, int co, int k, double omega,
+                       hipStream_t st);
+std::vector<int> run_launches(int n, int k);
 int x2_set_tune(int dtype, int edge, int wg, int zchunk);
 int x2_get_tune(int dtype, int edge, int *wg, int *zchunk);
 int autotune_x2(cnv_grid_s *u, cnv_grid_s *out, int iters, int *best_wg, int *best_z, double *results,

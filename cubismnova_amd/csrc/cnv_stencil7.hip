@@ -452,8 +452,7 @@ static int check_faces(cnv_grid_s *g, int comp)
 
 // State of one launch inside a multi-step run (cnv_diffusion_run).
 struct S7Run {
-    double *partials;          // this launch's partial buffer (first set)
-    double *partials2;         // second set (two-step launches)
+    double *partials;          // this launch's partial buffer
     const double *prev[2];     // the previous launch's partial sets, summed by workgroup 0
     int prev_n[2];
     double *prev_out[2];
@@ -627,80 +626,6 @@ int launch_diffusion_noalloc(const cnv_grid_desc *desc, const void *u, void *u_n
     if (rc != CNV_OK)
         return rc;
     return launch_stencil7_t(&gu, &go, nullptr, 0, 0, desc->ncomp, 1, nu_dt, sumsq, st, nullptr, nullptr, &scr);
-}
-
-// nsteps Euler steps alternating u -> tmp -> u ...  On grids of 16^3 or 32^3
-// blocks that are periodic or have walls of one rule each an even number of two-step launches covers the steps
-// up to a multiple of four, single steps the rest (so the field ends in u
-// for even nsteps, in tmp for odd).  The norms of a launch are reduced by
-// workgroup 0 of the next launch from the other half of u's partial buffer,
-// those of the last launch by k_finalize_sum.
-int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_dt, double *norms, hipStream_t st)
-{
-    double *P[2] = {u->partials, u->partials + u->partials_cap};
-    const size_t cap = u->partials_cap;
-    int nfused = 0, xwg = 0, xz = 0;
-    X2Faces faces[kX2MaxComp];
-    const bool periodic = nsteps >= 4 && !force_generic() && x2_applicable(u) && x2_applicable(tmp);
-    const bool walls = nsteps >= 4 && !force_generic() && !periodic && x2_walls(u, faces);
-    if (periodic || walls) {
-        x2_tile(u, &xwg, &xz);
-        if (2 * x2_tiles(u, xz) <= (long long)cap)
-            nfused = 2 * (nsteps / 4);
-    }
-    const double *prev[2] = {nullptr, nullptr};
-    int prev_n[2] = {0, 0};
-    double *prev_out[2] = {nullptr, nullptr};
-    int k = 0, L = 0; // steps and launches done
-    auto grid_at = [&](int l) { return l % 2 == 0 ? u : tmp; };
-    for (int j = 0; j < nfused; ++j, ++L) {
-        double *p1 = norms ? P[L % 2] : nullptr;
-        double *p2 = norms ? p1 + x2_tiles(u, xz) : nullptr;
-        int nt = 0;
-        const int rc = launch_diffusion_x2(grid_at(L), grid_at(L + 1), nu_dt, p1, p2, prev, prev_n, prev_out, xwg, xz,
-                                           &nt, st, walls ? faces : nullptr);
-        if (rc != CNV_OK)
-            return rc;
-        if (norms) {
-            prev[0] = p1;
-            prev[1] = p2;
-            prev_n[0] = prev_n[1] = nt;
-            prev_out[0] = norms + k;
-            prev_out[1] = norms + k + 1;
-        }
-        k += 2;
-    }
-    for (; k < nsteps; ++k, ++L) {
-        S7Run run;
-        run.partials = P[L % 2];
-        run.partials2 = nullptr;
-        for (int s = 0; s < 2; ++s) {
-            run.prev[s] = prev[s];
-            run.prev_n[s] = prev_n[s];
-            run.prev_out[s] = prev_out[s];
-        }
-        int nt = 0;
-        run.nparts = &nt;
-        run.cap = cap;
-        const int rc = launch_stencil7_t(grid_at(L), grid_at(L + 1), nullptr, 0, 0, u->desc.ncomp, 1, nu_dt,
-                                         norms ? norms + k : nullptr, st, nullptr, &run);
-        if (rc != CNV_OK)
-            return rc;
-        if (norms) {
-            prev[0] = P[L % 2];
-            prev[1] = nullptr;
-            prev_n[0] = nt;
-            prev_n[1] = 0;
-            prev_out[0] = norms + k;
-            prev_out[1] = nullptr;
-        }
-    }
-    for (int s = 0; s < 2; ++s)
-        if (prev[s]) {
-            hipLaunchKernelGGL(k_finalize_sum, dim3(1), dim3(1024), 0, st, prev[s], prev_n[s], prev_out[s]);
-            CNV_HIP(hipGetLastError());
-        }
-    return CNV_OK;
 }
 
 // ---------------------------------------------------------------- autotuner
@@ -1021,6 +946,118 @@ int launch_compare(const cnv_grid_s *a, int ca, const cnv_grid_s *b, int cb, dou
         compare_t<float, float>(a, ca, b, cb, partials, out, st);
     CNV_HIP(hipGetLastError());
     return CNV_OK;
+}
+
+// ---------------------------------------------------------------- multi-step runs
+
+// Steps per launch of a run: k at a time, then singles (k = 4: pairs too), in
+// as many launches as has the parity of n, so that the field ends in u for even
+// n and in tmp for odd.
+std::vector<int> run_launches(int n, int k)
+{
+    int c4 = 0, c2 = 0;
+    if (k == 2) {
+        c2 = 2 * (n / 4);
+    } else if (k == 4) {
+        c4 = n / 4;
+        const int rem = n % 4;
+        // launches so far plus those of the rest: 0, 1 (single), 1 (pair), 2 (pair, single)
+        if (rem < 2 && c4 % 2 != 0) {
+            --c4;
+            c2 = 2;
+        } else if (rem >= 2 && c4 % 2 != 0) {
+            c2 = 1;
+        }
+    }
+    std::vector<int> l(c4, 4);
+    l.insert(l.end(), c2, 2);
+    l.insert(l.end(), n - 4 * c4 - 2 * c2, 1);
+    return l;
+}
+
+// nsteps Euler steps alternating u -> tmp -> u ..., several per launch where
+// the grid is periodic or has walls of one rule each: four or two by LDS tiles
+// on small and medium grids (tile_steps), two by the z-marching kernel on larger
+// ones of 16^3 and 32^3 blocks.  A pinned tile of that kernel keeps it.
+// The norms of a launch are reduced by the next launch from the other half of
+// u's partial buffer, those of the last launch by a launch of their own.
+int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_dt, double *norms, hipStream_t st)
+{
+    double *P[2] = {u->partials, u->partials + u->partials_cap};
+    const size_t cap = u->partials_cap;
+    int xwg = 0, xz = 0, k = 1;
+    bool tiles = false;
+    X2Faces faces[kX2MaxComp];
+    bool periodic = false, walls = false;
+    if (nsteps >= 4 && !force_generic()) {
+        periodic = run_periodic(u) && run_periodic(tmp);
+        walls = !periodic && run_walls(u, faces);
+    }
+    if (periodic || walls) {
+        const int nc = u->desc.ncomp;
+        const bool x2 = x2_shape_ok(u);
+        const bool pinned = x2 && x2_tile(u, &xwg, &xz);
+        const int kt = pinned ? 0 : tile_steps(u, x2);
+        tiles = kt > 0 && (size_t)kt * tile_count(u, kt, nc) <= cap && (size_t)2 * tile_count(u, 2, nc) <= cap;
+        if (tiles)
+            k = kt;
+        else if (x2 && 2 * x2_tiles(u, xz) <= (long long)cap)
+            k = 2;
+    }
+    const double *prev = nullptr; // nprev sets of prev_n partials, consecutive
+    int nprev = 0, prev_n = 0;
+    double *prev_out = nullptr;
+    auto flush = [&]() -> int {
+        if (nprev > 0) {
+            hipLaunchKernelGGL(k_finalize_red, dim3(nprev), dim3(1024), 0, st, prev, prev_n, prev_out, -1);
+            CNV_HIP(hipGetLastError());
+        }
+        nprev = 0;
+        return CNV_OK;
+    };
+    int done = 0, L = 0; // steps and launches done
+    for (const int kk : run_launches(nsteps, k)) {
+        cnv_grid_s *a = L % 2 == 0 ? u : tmp, *b = L % 2 == 0 ? tmp : u;
+        double *part = norms ? P[L % 2] : nullptr;
+        int nt = 0, rc = CNV_OK;
+        if (kk > 1 && tiles) {
+            rc = launch_tile_euler(a, b, kk, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
+            nt = tile_count(u, kk, u->desc.ncomp);
+        } else {
+            if (nprev > 2)
+                rc = flush();
+            const double *pp[2] = {nprev > 0 ? prev : nullptr, nprev > 1 ? prev + prev_n : nullptr};
+            const int pn[2] = {prev_n, prev_n};
+            double *po[2] = {prev_out, prev_out + 1};
+            if (rc == CNV_OK && kk > 1) {
+                rc = launch_diffusion_x2(a, b, nu_dt, part, part ? part + x2_tiles(u, xz) : nullptr, pp, pn, po, xwg, xz,
+                                         &nt, st, walls ? faces : nullptr);
+            } else if (rc == CNV_OK) {
+                S7Run run;
+                run.partials = part;
+                for (int s = 0; s < 2; ++s) {
+                    run.prev[s] = pp[s];
+                    run.prev_n[s] = pn[s];
+                    run.prev_out[s] = po[s];
+                }
+                run.nparts = &nt;
+                run.cap = cap;
+                rc = launch_stencil7_t(a, b, nullptr, 0, 0, u->desc.ncomp, 1, nu_dt, norms ? norms + done : nullptr, st,
+                                       nullptr, &run);
+            }
+        }
+        if (rc != CNV_OK)
+            return rc;
+        if (norms) {
+            prev = part;
+            nprev = kk;
+            prev_n = nt;
+            prev_out = norms + done;
+        }
+        done += kk;
+        ++L;
+    }
+    return flush();
 }
 
 } // namespace cnv

@@ -645,7 +645,7 @@ bool x2_dispatch(int dtype, int edge, int wg, int zc, const X2Args &a, int ntile
 
 } // namespace
 
-static bool x2_shape_ok(const cnv_grid_s *u)
+bool x2_shape_ok(const cnv_grid_s *u)
 {
     const int *n = u->desc.block_cells;
     // the kernel addresses a component slab with 32-bit byte offsets
@@ -654,26 +654,35 @@ static bool x2_shape_ok(const cnv_grid_s *u)
 
 // The faces of every component of a grid with walls, each domain face of one
 // rule on all its blocks; false for other grids (they step one at a time).
-bool x2_walls(cnv_grid_s *u, X2Faces *faces)
+bool run_walls(cnv_grid_s *u, X2Faces *faces)
 {
-    if (!x2_shape_ok(u) || u->desc.ncomp > kX2MaxComp)
+    if (u->desc.ncomp > kX2MaxComp)
         return false;
-    for (int c = 0; c < u->desc.ncomp; ++c)
-        if (!jacobi2_faces(u, c, faces[c].fm, faces[c].fv))
+    std::lock_guard<std::mutex> lk(u->mtx);
+    for (int c = 0; c < u->desc.ncomp; ++c) {
+        const FaceInfo &f = face_info(u, c);
+        if (!f.uniform)
             return false;
+        for (int d = 0; d < 3; ++d)
+            for (int s = 0; s < 2; ++s) {
+                faces[c].fm[d][s] = f.fm[d][s];
+                faces[c].fv[d][s] = f.fv[d][s];
+            }
+    }
     return true;
 }
 
-bool x2_applicable(cnv_grid_s *u)
+// No block of the grid carries a BC.
+bool run_periodic(cnv_grid_s *u)
 {
-    if (!x2_shape_ok(u))
-        return false;
     std::lock_guard<std::mutex> lk(u->mtx);
     for (int c = 0; c < u->desc.ncomp; ++c)
         if (face_info(u, c).longest > 0)
             return false;
     return true;
 }
+
+bool x2_applicable(cnv_grid_s *u) { return x2_shape_ok(u) && run_periodic(u); }
 
 long long x2_tiles(const cnv_grid_s *u, int zchunk)
 {
@@ -749,7 +758,7 @@ int x2_get_tune(int dtype, int edge, int *wg, int *zchunk)
     return CNV_OK;
 }
 
-// The tile of a run on this grid: the pinned one, else the built-in workgroup
+// The tile of a run on this grid (true: pinned): the pinned one, else the built-in workgroup
 // size with the deepest z chunk that gives enough tiles, down to two planes.  A chunk of zc planes
 // marches zc + 2 planes one after another, each about 0.9 us (one barrier,
 // one exposed load), so on a small grid the chain is the launch: 64^3 FP64 in
@@ -757,7 +766,7 @@ int x2_get_tune(int dtype, int edge, int *wg, int *zchunk)
 // 128^3 FP32 in 32^3 blocks 9.4 / 6.0 / 5.0 / 5.0.  A shallow chunk reads and
 // evaluates more halo planes, which costs once the GPU is full: 256^3 FP32
 // 14.6 / 17.7 / 21.3 / 25.7, 192^3 FP64 13.1 / 15.5 / 18.0 / 21.6 in 32^3 blocks.
-void x2_tile(cnv_grid_s *u, int *wg, int *zchunk)
+bool x2_tile(cnv_grid_s *u, int *wg, int *zchunk)
 {
     const int dtype = u->desc.dtype, edge = u->desc.block_cells[0];
     bool pinned = false;
@@ -767,6 +776,7 @@ void x2_tile(cnv_grid_s *u, int *wg, int *zchunk)
             t.zchunk /= 2;
     *wg = t.wg;
     *zchunk = t.zchunk;
+    return pinned;
 }
 
 // Times every valid (workgroup size, z-planes per tile) pair of the two-step

@@ -235,11 +235,11 @@ int cnv_diffusion_step_noalloc(const cnv_grid_desc *desc, const void *u, void *u
  * BC lists as u.  If norms is non-NULL (device array of nsteps doubles)
  * norms[k] is the FP64 sum of squares after step k; the reductions of a
  * launch run inside the next launch (one finalize launch at the end).  On
- * grids of 16^3 or 32^3 blocks that are periodic (no BC list) or whose BC
- * lists give each domain face one rule on all its blocks (periodic on both
- * sides of an axis, or per side Dirichlet, Symmetry of nonzero sign or
- * Absorbing), steps go two per launch (one HBM read and write for two steps)
- * up to a multiple of four.  The loop of the reference's time stepping over Field.h:457-512 / FieldOperator.h. */
+ * grids that are periodic (no BC list) or whose BC lists give each domain face
+ * one rule on all its blocks (periodic on both sides of an axis, or per side
+ * Dirichlet, Symmetry of nonzero sign or Absorbing), runs of four steps and more
+ * go four or two steps per launch on small and medium grids of any block shape
+ * and two on every grid of 16^3 or 32^3 blocks.  The loop of the reference's time stepping over Field.h:457-512 / FieldOperator.h. */
 int cnv_diffusion_run(cnv_grid u, cnv_grid tmp, int nsteps, double nu_dt, double *norms, cnv_stream s);
 
 /* Fifth-order WENO face states (Jiang & Shu, J. Comput. Phys. 126:202-228,
@@ -490,8 +490,10 @@ int cnv_autotune_stencil7(cnv_grid u, cnv_grid out, int iters, int *wg, int *zch
                           int max_results, int *nresults);
 int cnv_tune_set_stencil7(int dtype, int edge, int wg, int zchunk);
 int cnv_tune_get_stencil7(int dtype, int edge, int *wg, int *zchunk);
-/* The same for the two-step kernel that cnv_diffusion_run uses on periodic
- * grids (no BC list on any block) of 16^3 or 32^3 blocks: `tmp` is
+/* The same for the two-step kernel that cnv_diffusion_run uses on grids of
+ * 16^3 or 32^3 blocks (on all of them where a tile other than the built-in one is
+ * set, else on those too large for its LDS tiles); timed on periodic grids (no BC
+ * list on any block): `tmp` is
  * overwritten; CNV_ERR_UNSUPPORTED for other grids. */
 int cnv_autotune_diffusion_run(cnv_grid u, cnv_grid tmp, int iters, int *wg, int *zchunk, double *results,
                                int max_results, int *nresults);

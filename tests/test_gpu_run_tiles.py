@@ -1,0 +1,51 @@
+"""Runs of several steps per launch on LDS tiles of the domain (block shapes
+outside 16^3 and 32^3): fields equal to single steps bit for bit, norms to 1e-13
+(another summation order), for every remainder of the step count, at shapes
+where tiles end inside blocks, blocks inside tiles, the domain inside a tile or
+its halo, and rows that no vector divides; components with walls of their own."""
+import numpy as np
+import pytest
+
+import cubismnova_amd as cnv
+from tests.helpers import assert_same, cells_of
+from tests.test_gpu_cols import MIXED, PARTLY, WALLS, build
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [((1, 1, 1), (5, 7, 3)), ((2, 3, 1), (6, 5, 33)), ((3, 3, 3), (8, 8, 8)), ((1, 2, 2), (24, 24, 24)),
+          ((2, 1, 2), (40, 13, 6)), ((1, 1, 3), (1, 1, 1)), ((2, 1, 1), (65, 64, 5)), ((17, 2, 2), (1, 3, 2)),
+          ((1, 2, 1), (64, 64, 64)), ((2, 2, 2), (16, 16, 12)), ((8, 7, 6), (8, 12, 16)), ((9, 10, 9), (12, 12, 12))]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+@pytest.mark.parametrize("walls", ["periodic", "three components"] + sorted(WALLS))
+def test_run_matches_single_steps(gpu, dtype, shape, walls):
+    nb, n = shape
+    lists = {"periodic": [[]], "three components": [MIXED, [], PARTLY]}.get(walls) or [WALLS[walls]]
+    u, _, _ = build(nb, n, dtype, 61, lists)
+    v, _, _ = build(nb, n, dtype, 61, lists)
+    t, _, _ = build(nb, n, dtype, 61, lists)
+    w, _, _ = build(nb, n, dtype, 61, lists)
+    dt = 0.1 / max(nb[d] * n[d] for d in range(3)) ** 2
+    a, b = v, w
+    for steps in (4, 5, 6, 7, 9):
+        norms, want = cnv.DeviceBuffer(8 * steps), cnv.DeviceBuffer(8 * steps)
+        norms.fill(np.float64, np.nan)
+        res = cnv.diffusion_run(u, t, steps, dt, norms)
+        assert res is (u if steps % 2 == 0 else t)
+        u, t = res, (t if res is u else u)
+        for k in range(steps):
+            cnv.diffusion_step(a, b, dt, sumsq=want.at(8 * k))
+            a, b = b, a
+        for c in range(len(lists)):
+            assert_same(cells_of(u.download(c), nb, n, u.block_stride), cells_of(a.download(c), nb, n, a.block_stride),
+                        "%d steps, component %d" % (steps, c))
+        gn, wn = norms.download(np.float64, steps), want.download(np.float64, steps)
+        assert np.max(np.abs(gn - wn) / wn) <= 1e-13
+    # without norms
+    u2 = cnv.diffusion_run(u, t, 4, dt)
+    for k in range(4):
+        cnv.diffusion_step(a, b, dt)
+        a, b = b, a
+    assert_same(cells_of(u2.download(0), nb, n, u.block_stride), cells_of(a.download(0), nb, n, a.block_stride))

@@ -1078,26 +1078,31 @@ int cnv_jacobi_solve(cnv_grid u, cnv_grid f, cnv_grid work, const cnv_solve_opts
     // values as single sweeps, u and f read once per pair)
     const bool two = refine ? jacobi2_applies(work, 0, work, work) && jacobi2_applies(work, 1, work, work)
                             : jacobi2_applies(u, 0, f, work) && jacobi2_applies(work, 0, f, u);
+    // the launches of a cycle: four sweeps each on small grids, else pairs; the
+    // plain cycle ends in u (an even number of launches), the refined one in
+    // either correction component
+    const int kmax = !two ? 1 : jacobi2_tile_sweeps(refine ? work : u) == 4 ? 4 : 2;
+    std::vector<int> plan = run_launches(S, kmax);
+    if (refine && kmax > 1) {
+        plan.assign(S / kmax, kmax);
+        if (S % kmax)
+            plan.push_back(S % kmax); // two sweeps left over by fours
+    }
+    auto sweeps_of = [&](int k, cnv_grid_s *a, int ca, cnv_grid_s *r, int cr, cnv_grid_s *b, int cb) -> int {
+        if (k == 4)
+            return launch_tile_jacobi(a, ca, r, cr, b, cb, 4, o->omega, st);
+        return k == 2 ? launch_jacobi2(a, ca, r, cr, b, cb, o->omega, st, nullptr)
+                      : launch_jacobi(a, ca, r, cr, b, cb, 0, o->omega, nullptr, st);
+    };
     auto cycle = [&]() -> int {
-        int crc = CNV_OK;
-        if (refine) {
-            crc = launch_fill((char *)work->data, CNV_F32, 0.0, work->component_bytes / 4, st);
-            const int L = two ? S / 2 : S;
-            for (int k = 0; k < L && crc == CNV_OK; ++k)
-                crc = two ? launch_jacobi2(work, k % 2, work, 2, work, 1 - k % 2, o->omega, st, nullptr)
-                          : launch_jacobi(work, k % 2, work, 2, work, 1 - k % 2, 0, o->omega, nullptr, st);
-            if (crc == CNV_OK)
-                crc = launch_correct(u, 0, work, L % 2, st);
-        } else {
-            // an even number of pair launches (u -> work -> u ...), then the
-            // remaining two sweeps, if any, one at a time: the cycle ends in u
-            const int pairs = two ? (S / 2) & ~1 : 0;
-            for (int k = 0; k < pairs + (S - 2 * pairs) && crc == CNV_OK; ++k) {
-                cnv_grid_s *a = k % 2 == 0 ? u : work, *b = k % 2 == 0 ? work : u;
-                crc = k < pairs ? launch_jacobi2(a, 0, f, 0, b, 0, o->omega, st, nullptr)
-                                : launch_jacobi(a, 0, f, 0, b, 0, 0, o->omega, nullptr, st);
-            }
+        int crc = refine ? launch_fill((char *)work->data, CNV_F32, 0.0, work->component_bytes / 4, st) : CNV_OK;
+        for (size_t i = 0; i < plan.size() && crc == CNV_OK; ++i) {
+            const int p = (int)(i % 2);
+            crc = refine ? sweeps_of(plan[i], work, p, work, 2, work, 1 - p)
+                         : sweeps_of(plan[i], p == 0 ? u : work, 0, f, 0, p == 0 ? work : u, 0);
         }
+        if (crc == CNV_OK && refine)
+            crc = launch_correct(u, 0, work, (int)(plan.size() % 2), st);
         return crc == CNV_OK ? defect() : crc;
     };
     rc = launch_sums(f, 0, hst, st);

@@ -826,6 +826,25 @@ bool jacobi2_applies(cnv_grid_s *u, int cu, cnv_grid_s *f, cnv_grid_s *out)
     return jacobi2_faces(u, cu, fm, fv);
 }
 
+// Sweeps per LDS tile launch of a grid that takes the two-sweep kernel; 0: that
+// kernel (always where its tile is pinned).  us per sweep, this kernel / tiles of
+// four / of two, Dirichlet faces: 64^3 in 32^3 blocks 4.5 / 2.4 / 3.8 FP32, 4.7 / 2.8
+// / 4.4 FP64; 80^3 in 16^3 4.3 / 3.1 / 4.0 FP32, 4.8 / 5.0 / 4.7 FP64; 96^3 in 32^3
+// 5.3 / 5.0 / 4.6 FP32, 5.7 / 8.4 / 7.6 FP64; 128^3 in 64^3 6.7 / 8.8 / 8.4 FP32.  So
+// fours while every tile has its place on the GPU at once (one per CU in FP64,
+// whose three LDS arrays take 149 KB, two in FP32), then pairs of FP32 up to 96^3.
+int jacobi2_tile_sweeps(const cnv_grid_s *u)
+{
+    bool pinned = false;
+    (void)j2_tune(u->desc.dtype, u->desc.block_cells[0], &pinned);
+    const int t4 = tile_count(u, 4, 1), t2 = tile_count(u, 2, 1);
+    if (pinned || t4 == 0 || t2 == 0)
+        return 0;
+    if (u->desc.dtype == CNV_F64)
+        return t4 <= 256 ? 4 : 0;
+    return t4 <= 512 ? 4 : t2 <= 450 ? 2 : 0;
+}
+
 int launch_jacobi2(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out, int co, double omega,
                    hipStream_t st, const int *tile)
 {
@@ -844,6 +863,9 @@ int launch_jacobi2(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out
         if (rc != CNV_OK)
             return rc;
     }
+    // (FP64 pairs: 4.0-4.7 us per sweep here, 4.3-4.7 on tiles)
+    if (!tile && u->desc.dtype == CNV_F32 && jacobi2_tile_sweeps(u) > 0)
+        return launch_tile_jacobi(u, cu, f, cf, out, co, 2, omega, st);
     a.u = static_cast<const char *>(u->data);
     a.f = static_cast<const char *>(f->data);
     a.out = static_cast<char *>(out->data);

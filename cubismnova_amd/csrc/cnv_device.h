@@ -118,6 +118,16 @@ __device__ inline void buf_store(__amdgpu_buffer_rsrc_t r, unsigned voff, unsign
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, x), r, (int)voff, (int)soff, 0);
 }
 
+template <typename T>
+__device__ inline void buf_store1(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, T v)
+{
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    if constexpr (sizeof(T) == 4)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)voff, (int)soff, 0);
+    else
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)voff, (int)soff, 0);
+}
+
 // Streaming (non-temporal) vector load of exactly N elements, for data read
 // once per launch.
 template <typename T, int N>

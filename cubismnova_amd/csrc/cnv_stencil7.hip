@@ -977,8 +977,9 @@ std::vector<int> run_launches(int n, int k)
 
 // nsteps Euler steps alternating u -> tmp -> u ..., several per launch where
 // the grid is periodic or has walls of one rule each: four or two by LDS tiles
-// on small and medium grids (tile_steps), two by the z-marching kernel on larger
-// ones of 16^3 and 32^3 blocks.  A pinned tile of that kernel keeps it.
+// on small grids (tile_steps), two on larger ones by the kernels that march through
+// z, on tiles of blocks of 16^3 and 32^3 cells or of the domain.  A pinned tile of
+// the former keeps it.
 // The norms of a launch are reduced by the next launch from the other half of
 // u's partial buffer, those of the last launch by a launch of their own.
 int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_dt, double *norms, hipStream_t st)
@@ -987,6 +988,7 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
     const size_t cap = u->partials_cap;
     int xwg = 0, xz = 0, k = 1;
     bool tiles = false;
+    int rz = 0, nt2 = 0;
     X2Faces faces[kX2MaxComp];
     bool periodic = false, walls = false;
     if (nsteps >= 4 && !force_generic()) {
@@ -995,14 +997,22 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
     }
     if (periodic || walls) {
         const int nc = u->desc.ncomp;
-        const bool x2 = x2_shape_ok(u);
-        const bool pinned = x2 && x2_tile(u, &xwg, &xz);
-        const int kt = pinned ? 0 : tile_steps(u, x2);
+        const bool shape = x2_shape_ok(u), pinned = shape && x2_tile(u, &xwg, &xz);
+        // the block-marching kernel, whose halo is the cheaper one, but for FP32 on
+        // 16^3 blocks (us per step, block / domain tiles: 112^3 6.3 / 4.9, 256^3 21.8
+        // / 17.2, with walls 27.1 / 22.9; 256^3 FP32 in 32^3 14.6 / 17.4, FP64 24.4 /
+        // 34.9, in 16^3 FP64 30.3 / 34.1)
+        const bool x2 = shape && (pinned || u->desc.dtype == CNV_F64 || u->desc.block_cells[0] == 32);
+        const int kt = pinned ? 0 : tile_steps(u, x2, walls);
         tiles = kt > 0 && (size_t)kt * tile_count(u, kt, nc) <= cap && (size_t)2 * tile_count(u, 2, nc) <= cap;
-        if (tiles)
+        if (tiles) {
             k = kt;
-        else if (x2 && 2 * x2_tiles(u, xz) <= (long long)cap)
-            k = 2;
+        } else if (x2) {
+            k = 2 * x2_tiles(u, xz) <= (long long)cap ? 2 : 1;
+        } else {
+            nt2 = run2_tiles(u, &rz);
+            k = nt2 > 0 && (size_t)2 * nt2 <= cap ? 2 : 1;
+        }
     }
     const double *prev = nullptr; // nprev sets of prev_n partials, consecutive
     int nprev = 0, prev_n = 0;
@@ -1023,6 +1033,9 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
         if (kk > 1 && tiles) {
             rc = launch_tile_euler(a, b, kk, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
             nt = tile_count(u, kk, u->desc.ncomp);
+        } else if (kk > 1 && nt2 > 0) {
+            rc = launch_run2(a, b, rz, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
+            nt = nt2;
         } else {
             if (nprev > 2)
                 rc = flush();

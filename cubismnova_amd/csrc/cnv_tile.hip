@@ -2,8 +2,7 @@
 // the domain held in LDS, for any block shape.
 //
 // On small grids a launch costs about 4.5 us whatever it does, and the
-// plane-marching kernels add a serial chain of planes; on block shapes outside
-// 16^3 and 32^3 only single steps exist.  Here a workgroup loads a tile of
+// plane-marching kernels add a serial chain of planes.  Here a workgroup loads a tile of
 // CX x CY x CZ cells of the domain, wherever its blocks lie, plus K cells on
 // every side into LDS, evaluates step j on the cells within K - j of the tile
 // (so that step K covers exactly the tile), and writes the tile.  Block
@@ -361,29 +360,29 @@ int tile_count(const cnv_grid_s *u, int k, int ncomp)
     return ok ? a.ntiles : 0;
 }
 
-// Euler steps per tile launch on u where the alternative is `marching` (the
-// z-marching two-step kernel) or single steps; 0: the alternative.  Figures are
-// us per step of runs with norms, alternative / tiles.  Four steps while there is
-// at most one tile per CU, where the launch is its fixed 4.5 us plus one tile's
-// 5 us (64^3 in 32^3 blocks 3.5 / 2.4 FP32, 4.0 / 3.1 FP64, with walls 4.5 / 2.9
-// and 4.6 / 3.5; 60^3 in 20^3 blocks 4.5 / 2.4 and 4.8 / 3.1); with more, the 2.2
-// evaluations per cell of four steps cost more than the launches of two (80^3
-// FP32: 3.5 with four, 3.2 with two).  Two steps up to 1100 tiles against single
-// steps (72^3 in 12^3 blocks 4.6 / 3.2 FP32, 5.1 / 3.9 FP64, 128^3 in 64^3 blocks
-// 9.2 / 7.6 and 9.6 / 8.9, 144^3 FP64 15.2 / 14.2; 192^3 FP32 13.9 / 15.7); in FP32
-// up to 450 against the marching kernel, whose tiles are then too few (16^3
-// blocks: 80^3 4.2 / 3.2, 96^3 5.0 / 4.0, with walls 6.1 / 4.5; 96^3 in 32^3 blocks
-// 3.9 / 4.1), not in FP64 (80^3 4.3 / 4.2, 96^3 5.2 / 5.4).
-int tile_steps(const cnv_grid_s *u, bool marching)
+// Euler steps per tile launch on u; 0: the kernels that march through z take it,
+// two steps per launch, on tiles of blocks (`block_tiles`) or of the domain.
+// Figures are us per step of runs with norms, marching / tiles.  Four steps while
+// there is at most one tile per CU, where the launch is its fixed 4.5 us plus one
+// tile's 5 us (64^3 in 32^3 blocks 3.5 / 2.4 FP32, 4.0 / 3.1 FP64, with walls 4.5 /
+// 2.9 and 4.6 / 3.5; 60^3 in 20^3 blocks, against single steps, 4.5 / 2.4 and 4.8
+// / 3.1); with more, the 2.2 evaluations per cell of four steps cost more than
+// the launches of two (80^3 FP32: 3.5 with four, 3.2 with two).  Two steps while
+// the marching kernels have too few tiles.  In FP32, against domain tiles up to
+// 500 tiles (72^3 3.6 / 3.2, 108^3 4.2 / 5.0), with walls, which cost those more, up
+// to 700 (96^3 5.1 / 4.5, 108^3 6.3 / 5.7, 120^3 periodic 5.7 / 6.4); against block
+// tiles up to 450 (96^3 in 32^3 blocks 4.1 / 3.9).  In FP64, against domain tiles
+// up to 450 (72^3 3.85 / 3.85, 96^3 with walls 5.9 / 5.7, 120^3 6.1 / 8.9).
+int tile_steps(const cnv_grid_s *u, bool block_tiles, bool walls)
 {
     const int t4 = tile_count(u, 4, u->desc.ncomp), t2 = tile_count(u, 2, u->desc.ncomp);
     if (t4 == 0 || t2 == 0)
         return 0;
     if (t4 <= 256)
         return 4;
-    if (marching)
-        return u->desc.dtype == CNV_F32 && t2 <= 450 ? 2 : 0;
-    return t2 <= 1100 ? 2 : 0;
+    const bool f32 = u->desc.dtype == CNV_F32;
+    const int most = block_tiles ? (f32 ? 450 : 0) : f32 ? (walls ? 700 : 500) : 450;
+    return t2 <= most ? 2 : 0;
 }
 
 int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int k, double nu_dt, double *part, const double *prev_p,

@@ -268,7 +268,7 @@ bool x2_shape_ok(const cnv_grid_s *u);
 bool x2_applicable(cnv_grid_s *u);
 long long x2_tiles(const cnv_grid_s *u, int zchunk);
 bool x2_tile(cnv_grid_s *u, int *wg, int *zchunk);
-int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *part1, double *part2,
+int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, double nu_dt, double *part1, double *part2,
                         const double *const prev_p[2], const int prev_n[2], double *const prev_out[2], int wg,
                         int zchunk, int *nparts, hipStream_t st, const X2Faces *faces = nullptr);
 // 2 or 4 Euler steps or Jacobi sweeps per launch on LDS tiles of the domain, any
@@ -276,7 +276,7 @@ int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *pa
 // another kernel), the launches; the launches of n steps, up to k at a time
 int tile_count(const cnv_grid_s *u, int k, int ncomp);
 int tile_steps(const cnv_grid_s *u, bool block_tiles, bool walls);
-int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int k, double nu_dt, double *part, const double *prev_p,
+int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int k, double nu_dt, double *part, const double *prev_p,
                       int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st);
 int launch_tile_jacobi(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out, int co, int k, double omega,
                        hipStream_t st);
@@ -284,8 +284,8 @@ std::vector<int> run_launches(int n, int k);
 // two Euler steps per launch on domain tiles that march through z, any block
 // shape (cnv_run2.hip): tiles (0: not available) and planes per tile; the launch
 int run2_tiles(const cnv_grid_s *u, int *zchunk);
-int launch_run2(cnv_grid_s *u, cnv_grid_s *out, int zchunk, double nu_dt, double *part, const double *prev_p, int nprev,
-                int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st);
+int launch_run2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int zchunk, double nu_dt, double *part, const double *prev_p,
+                int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st);
 int x2_set_tune(int dtype, int edge, int wg, int zchunk);
 int x2_get_tune(int dtype, int edge, int *wg, int *zchunk);
 int autotune_x2(cnv_grid_s *u, cnv_grid_s *out, int iters, int *best_wg, int *best_z, double *results,

@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kRun2WG) void k_run2(const Run2Args a)
 // ---------------------------------------------------------------- host side
 
 template <typename T>
-static bool run2_layout(const cnv_grid_s *u, Run2Args &a, int zchunk)
+static bool run2_layout(const cnv_grid_s *u, Run2Args &a, int ncomp, int zchunk)
 {
     constexpr int VEC = 16 / (int)sizeof(T), CX = 14 * VEC, CY = kRun2WG / 16 - 4;
     const Geom G = geom_of(u);
@@ -330,7 +330,7 @@ static bool run2_layout(const cnv_grid_s *u, Run2Args &a, int zchunk)
         return false;
     a.bstride = (unsigned)u->block_bytes;
     const int c[3] = {CX, CY, zchunk};
-    long long nt = u->desc.ncomp;
+    long long nt = ncomp;
     for (int d = 0; d < 3; ++d) {
         a.nb[d] = G.nb[d];
         a.n[d] = G.n[d];
@@ -367,7 +367,8 @@ static void run2_launch(const Run2Args &a, bool wall, hipStream_t st)
 static int run2_count(const cnv_grid_s *u, int zchunk)
 {
     Run2Args a;
-    const bool ok = u->desc.dtype == CNV_F64 ? run2_layout<double>(u, a, zchunk) : run2_layout<float>(u, a, zchunk);
+    const bool ok = u->desc.dtype == CNV_F64 ? run2_layout<double>(u, a, u->desc.ncomp, zchunk)
+                                             : run2_layout<float>(u, a, u->desc.ncomp, zchunk);
     return ok ? a.ntiles : 0;
 }
 
@@ -389,18 +390,18 @@ int run2_tiles(const cnv_grid_s *u, int *zchunk)
     return run2_count(u, *zchunk);
 }
 
-int launch_run2(cnv_grid_s *u, cnv_grid_s *out, int zchunk, double nu_dt, double *part, const double *prev_p, int nprev,
-                int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st)
+int launch_run2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int zchunk, double nu_dt, double *part, const double *prev_p,
+                int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st)
 {
     Run2Args a{};
     const bool f64 = u->desc.dtype == CNV_F64;
-    if (!(f64 ? run2_layout<double>(u, a, zchunk) : run2_layout<float>(u, a, zchunk)))
+    if (!(f64 ? run2_layout<double>(u, a, ncomp, zchunk) : run2_layout<float>(u, a, ncomp, zchunk)))
         return fail(CNV_ERR_UNSUPPORTED, "grid too large for two steps per launch");
     a.u = static_cast<const char *>(u->data);
     a.out = static_cast<char *>(out->data);
     a.cs_u = (long long)u->component_bytes;
     a.cs_o = (long long)out->component_bytes;
-    for (int c = 0; faces && c < u->desc.ncomp; ++c)
+    for (int c = 0; faces && c < ncomp; ++c)
         a.faces[c] = faces[c];
     for (int d = 0; d < 3; ++d)
         a.ih2[d] = 1. / (u->h[d] * u->h[d]);

@@ -986,6 +986,7 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
 {
     double *P[2] = {u->partials, u->partials + u->partials_cap};
     const size_t cap = u->partials_cap;
+    const int nc = u->desc.ncomp; // (tmp may have more)
     int xwg = 0, xz = 0, k = 1;
     bool tiles = false;
     int rz = 0, nt2 = 0;
@@ -996,7 +997,6 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
         walls = !periodic && run_walls(u, faces);
     }
     if (periodic || walls) {
-        const int nc = u->desc.ncomp;
         const bool shape = x2_shape_ok(u), pinned = shape && x2_tile(u, &xwg, &xz);
         // the block-marching kernel, whose halo is the cheaper one, but for FP32 on
         // 16^3 blocks (us per step, block / domain tiles: 112^3 6.3 / 4.9, 256^3 21.8
@@ -1031,10 +1031,10 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
         double *part = norms ? P[L % 2] : nullptr;
         int nt = 0, rc = CNV_OK;
         if (kk > 1 && tiles) {
-            rc = launch_tile_euler(a, b, kk, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
-            nt = tile_count(u, kk, u->desc.ncomp);
+            rc = launch_tile_euler(a, b, nc, kk, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
+            nt = tile_count(u, kk, nc);
         } else if (kk > 1 && nt2 > 0) {
-            rc = launch_run2(a, b, rz, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
+            rc = launch_run2(a, b, nc, rz, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
             nt = nt2;
         } else {
             if (nprev > 2)
@@ -1043,8 +1043,8 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
             const int pn[2] = {prev_n, prev_n};
             double *po[2] = {prev_out, prev_out + 1};
             if (rc == CNV_OK && kk > 1) {
-                rc = launch_diffusion_x2(a, b, nu_dt, part, part ? part + x2_tiles(u, xz) : nullptr, pp, pn, po, xwg, xz,
-                                         &nt, st, walls ? faces : nullptr);
+                rc = launch_diffusion_x2(a, b, nc, nu_dt, part, part ? part + x2_tiles(u, xz) : nullptr, pp, pn, po,
+                                         xwg, xz, &nt, st, walls ? faces : nullptr);
             } else if (rc == CNV_OK) {
                 S7Run run;
                 run.partials = part;
@@ -1055,7 +1055,7 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
                 }
                 run.nparts = &nt;
                 run.cap = cap;
-                rc = launch_stencil7_t(a, b, nullptr, 0, 0, u->desc.ncomp, 1, nu_dt, norms ? norms + done : nullptr, st,
+                rc = launch_stencil7_t(a, b, nullptr, 0, 0, nc, 1, nu_dt, norms ? norms + done : nullptr, st,
                                        nullptr, &run);
             }
         }

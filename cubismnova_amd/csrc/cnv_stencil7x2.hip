@@ -691,7 +691,7 @@ long long x2_tiles(const cnv_grid_s *u, int zchunk)
     return u->nblocks_total * u->desc.ncomp * ((edge + zc - 1) / zc);
 }
 
-int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *part1, double *part2,
+int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, double nu_dt, double *part1, double *part2,
                         const double *const prev_p[2], const int prev_n[2], double *const prev_out[2], int wg,
                         int zchunk, int *nparts, hipStream_t st, const X2Faces *faces)
 {
@@ -721,10 +721,10 @@ int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, double nu_dt, double *pa
         a.prev_n[k] = prev_n ? prev_n[k] : 0;
         a.prev_out[k] = prev_out ? prev_out[k] : nullptr;
     }
-    const long long ntiles = (long long)a.tiles_per_comp * u->desc.ncomp;
+    const long long ntiles = (long long)a.tiles_per_comp * ncomp;
     if (ntiles >= (1LL << 31))
         return fail(CNV_ERR_UNSUPPORTED, "grid too large for the two-step kernel");
-    for (int c = 0; faces && c < u->desc.ncomp; ++c)
+    for (int c = 0; faces && c < ncomp; ++c)
         a.faces[c] = faces[c];
     if (!(faces ? x2_dispatch_wall(u->desc.dtype, edge, zchunk, a, (int)ntiles, st)
                 : x2_dispatch(u->desc.dtype, edge, wg, zchunk, a, (int)ntiles, st)))
@@ -797,13 +797,13 @@ int autotune_x2(cnv_grid_s *u, cnv_grid_s *out, int iters, int *best_wg, int *be
         for (int z = 8; z <= edge && rc == CNV_OK; z *= 2) {
             if (x2_set_tune(u->desc.dtype, edge, wgs[wi], z) != CNV_OK)
                 continue;
-            rc = launch_diffusion_x2(u, out, 1e-9, nullptr, nullptr, nullptr, nullptr, nullptr, wgs[wi], z, nullptr,
+            rc = launch_diffusion_x2(u, out, u->desc.ncomp, 1e-9, nullptr, nullptr, nullptr, nullptr, nullptr, wgs[wi], z, nullptr,
                                      st);
             if (rc != CNV_OK)
                 break;
             (void)hipEventRecord(e0, st);
             for (int i = 0; i < iters && rc == CNV_OK; ++i)
-                rc = launch_diffusion_x2(u, out, 1e-9, nullptr, nullptr, nullptr, nullptr, nullptr, wgs[wi], z,
+                rc = launch_diffusion_x2(u, out, u->desc.ncomp, 1e-9, nullptr, nullptr, nullptr, nullptr, nullptr, wgs[wi], z,
                                          nullptr, st);
             (void)hipEventRecord(e1, st);
             if (hipEventSynchronize(e1) != hipSuccess) {

@@ -385,18 +385,18 @@ int tile_steps(const cnv_grid_s *u, bool block_tiles, bool walls)
     return t2 <= most ? 2 : 0;
 }
 
-int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int k, double nu_dt, double *part, const double *prev_p,
+int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int k, double nu_dt, double *part, const double *prev_p,
                       int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st)
 {
     TileArgs a{};
-    if (!(k == 2 ? tile_layout<2>(u, a, u->desc.ncomp) : tile_layout<4>(u, a, u->desc.ncomp)))
+    if (!(k == 2 ? tile_layout<2>(u, a, ncomp) : tile_layout<4>(u, a, ncomp)))
         return fail(CNV_ERR_UNSUPPORTED, "grid too large for the tile kernel");
     a.u = static_cast<const char *>(u->data);
     a.out = static_cast<char *>(out->data);
     a.cs_u = (long long)(u->component_bytes / u->elem);
     a.cs_o = (long long)(out->component_bytes / out->elem);
     bool wall = false;
-    for (int c = 0; faces && c < u->desc.ncomp; ++c) {
+    for (int c = 0; faces && c < ncomp; ++c) {
         a.faces[c] = faces[c];
         wall = true;
     }

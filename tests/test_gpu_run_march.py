@@ -47,3 +47,29 @@ def test_run_matches_single_steps(gpu, dtype, shape, walls):
         cnv.diffusion_step(a, b, dt)
         a, b = b, a
     assert_same(cells_of(t.download(0), nb, n, t.block_stride), cells_of(a.download(0), nb, n, a.block_stride))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("nb,n", [((6, 6, 6), (64, 64, 64)), ((24, 24, 24), (16, 16, 16)), ((19, 19, 19), (20, 20, 20))],
+                         ids=str)
+@pytest.mark.parametrize("walls", ["periodic", "mixed"])
+def test_several_rounds_of_workgroups(gpu, dtype, nb, n, walls):
+    """Grids whose tiles do not fit the GPU at once: equal to single steps in
+    every cell (compared on the device)."""
+    N = [nb[d] * n[d] for d in range(3)]
+    x = np.random.default_rng(71).standard_normal((N[2], N[1], N[0]), dtype=np.float32).astype(dtype)
+    grids = [cnv.Cartesian(nb, n, dtype=dtype) for _ in range(4)]
+    for g in grids:
+        for (k, d, s, v) in (WALLS[walls] if walls != "periodic" else []):
+            g.addFaceBC({1: cnv.Absorbing(d, s), 2: cnv.Dirichlet(d, s, v), 3: cnv.Symmetry(d, s, v)}[k])
+    u, t, a, b = grids
+    u.upload_global(0, x)
+    a.upload_global(0, x)
+    dt = 0.1 / max(N) ** 2
+    for rep in range(3):
+        assert cnv.diffusion_run(u, t, 8, dt) is u
+        for k in range(8):
+            cnv.diffusion_step(a, b, dt)
+            a, b = b, a
+        diff = cnv.grid_compare(u, a)
+        assert diff[0] == 0.0 and diff[2] == 0.0, diff

@@ -49,3 +49,53 @@ def test_run_matches_single_steps(gpu, dtype, shape, walls):
         cnv.diffusion_step(a, b, dt)
         a, b = b, a
     assert_same(cells_of(u2.download(0), nb, n, u.block_stride), cells_of(a.download(0), nb, n, a.block_stride))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("walls", [False, True])
+@pytest.mark.parametrize("nb,n", [((2, 2, 2), (20, 20, 20)), ((5, 5, 5), (24, 24, 24)), ((6, 5, 4), (32, 32, 32))],
+                         ids=str)
+def test_run_with_a_wider_second_grid(gpu, dtype, walls, nb, n):
+    """tmp may have more components than u: only u's are stepped, in the launches
+    that read tmp too."""
+    lists = [MIXED if walls else []]
+    u, _, _ = build(nb, n, dtype, 73, lists)
+    a, _, _ = build(nb, n, dtype, 73, lists)
+    b, _, _ = build(nb, n, dtype, 73, lists)
+    t, _, _ = build(nb, n, dtype, 79, lists * 3)
+    before = [t.download(c) for c in (1, 2)]
+    dt = 0.1 / max(nb[d] * n[d] for d in range(3)) ** 2
+    norms, want = cnv.DeviceBuffer(8 * 8), cnv.DeviceBuffer(8 * 8)
+    assert cnv.diffusion_run(u, t, 8, dt, norms) is u
+    for k in range(8):
+        cnv.diffusion_step(a, b, dt, sumsq=want.at(8 * k))
+        a, b = b, a
+    assert_same(cells_of(u.download(0), nb, n, u.block_stride), cells_of(a.download(0), nb, n, a.block_stride))
+    gn, wn = norms.download(np.float64, 8), want.download(np.float64, 8)
+    assert np.max(np.abs(gn - wn) / wn) <= 1e-13
+    for c in (1, 2):
+        assert_same(t.download(c), before[c - 1], "component %d of tmp" % c)
+
+
+@pytest.mark.parametrize("nb,n", [((2, 2, 2), (32, 32, 32)), ((5, 5, 5), (24, 24, 24))], ids=str)
+def test_captured_run(gpu, nb, n):
+    """A recorded run replays to the eager run's field and norms."""
+    u, _, _ = build(nb, n, np.float32, 83, [MIXED])
+    v, _, _ = build(nb, n, np.float32, 83, [MIXED])
+    t, _, _ = build(nb, n, np.float32, 83, [MIXED])
+    r, _, _ = build(nb, n, np.float32, 83, [MIXED])  # v's own second grid: the first two runs overlap
+    dt = 0.1 / max(nb[d] * n[d] for d in range(3)) ** 2
+    norms, want = cnv.DeviceBuffer(8 * 12), cnv.DeviceBuffer(8 * 12)
+    s = cnv.Stream()
+    cnv.diffusion_run(u, t, 12, dt, norms, stream=s)
+    cnv.diffusion_run(v, r, 12, dt, want)
+    s.synchronize()
+    g = cnv.Graph(s).capture()
+    cnv.diffusion_run(u, t, 12, dt, norms, stream=s)
+    g.end()
+    for rep in range(3):
+        g.launch()
+        s.synchronize()
+        cnv.diffusion_run(v, r, 12, dt, want)
+        assert_same(cells_of(u.download(0), nb, n, u.block_stride), cells_of(v.download(0), nb, n, v.block_stride))
+        assert np.array_equal(norms.download(np.float64, 12), want.download(np.float64, 12))

@@ -2,6 +2,7 @@
 // objects, BC lists and argument checking in front of the kernels.
 #include "cnv_internal.h"
 
+#include <memory>
 #include <cstdio>
 #include <cstring>
 #include <new>
@@ -57,27 +58,30 @@ int ensure_bc_table(cnv_grid_s *g, int comp)
         return CNV_OK;
     }
     const long long nb = g->nblocks_total;
-    std::vector<DevBCHead> heads((size_t)nb);
-    std::vector<DevBC> entries;
-    bool any = false;
+    size_t ne = 0;
+    for (const auto &l : g->bcs[comp])
+        ne += l.size();
+    // heads and entries in one image, written once
+    const size_t hb = sizeof(DevBCHead) * (size_t)nb, eb = sizeof(DevBC) * ne;
+    std::unique_ptr<char[]> image(new char[hb + eb]);
+    DevBCHead *const heads = reinterpret_cast<DevBCHead *>(image.get());
+    DevBC *const entries = reinterpret_cast<DevBC *>(image.get() + hb);
+    int at = 0;
     for (long long b = 0; b < nb; ++b) {
         const auto &lst = g->bcs[comp][(size_t)b];
-        heads[(size_t)b].offset = (int)entries.size();
-        heads[(size_t)b].count = (int)lst.size();
-        for (const auto &bc : lst) {
-            entries.push_back({bc.kind, bc.dir, bc.side, 0, bc.value});
-            any = true;
-        }
+        DevBCHead &h = heads[b];
+        h.offset = at;
+        h.count = (int)lst.size();
+        for (const auto &bc : lst)
+            entries[at++] = {bc.kind, bc.dir, bc.side, 0, bc.value};
         const int sb[3] = {-1, -1, -1}, se[3] = {2, 2, 2};
-        resolve_faces(entries.data() + heads[(size_t)b].offset, (int)lst.size(), sb, se, heads[(size_t)b].kind,
-                      heads[(size_t)b].val);
+        resolve_faces(entries + h.offset, h.count, sb, se, h.kind, h.val);
     }
     if (t.heads) {
         // the table is rewritten (BC lists changed): kernels still queued on
         // any stream may read it, so they finish first
         CNV_HIP(hipDeviceSynchronize());
     }
-    const size_t hb = sizeof(DevBCHead) * (size_t)nb, eb = sizeof(DevBC) * entries.size();
     if (hb + eb > t.bytes_cap) {
         if (t.heads)
             CNV_HIP(hipFree(t.heads));
@@ -87,12 +91,8 @@ int ensure_bc_table(cnv_grid_s *g, int comp)
         t.bytes_cap = hb + eb;
     }
     t.entries = reinterpret_cast<DevBC *>(reinterpret_cast<char *>(t.heads) + hb);
-    std::vector<char> image(hb + eb);
-    std::memcpy(image.data(), heads.data(), hb);
-    if (eb)
-        std::memcpy(image.data() + hb, entries.data(), eb);
-    CNV_HIP(hipMemcpy(t.heads, image.data(), hb + eb, hipMemcpyHostToDevice));
-    t.any = any;
+    CNV_HIP(hipMemcpy(t.heads, image.get(), hb + eb, hipMemcpyHostToDevice));
+    t.any = ne > 0;
     t.version = g->bc_version;
     return CNV_OK;
 }

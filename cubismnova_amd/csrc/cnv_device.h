@@ -112,8 +112,13 @@ __device__ inline void buf_store(__amdgpu_buffer_rsrc_t r, unsigned voff, unsign
 #pragma unroll
     for (int i = 0; i < N; ++i)
         x[i] = v.v[i];
+    // The uniform offset of a 16-byte store goes through the lane's register: with
+    // it in the instruction's scalar offset the compiler lets the next instruction
+    // overwrite the data registers (it assumes no hazard in that form; without a
+    // scalar offset it keeps the required distance), and a store followed so by
+    // a write of its third register has stored that register's new value in some lanes.
     if constexpr (sizeof(T) * N == 16)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, (int)voff, (int)soff, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, x), r, (int)(voff + soff), 0, 0);
     else
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, x), r, (int)voff, (int)soff, 0);
 }

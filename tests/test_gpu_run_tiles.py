@@ -99,3 +99,32 @@ def test_captured_run(gpu, nb, n):
         cnv.diffusion_run(v, r, 12, dt, want)
         assert_same(cells_of(u.download(0), nb, n, u.block_stride), cells_of(v.download(0), nb, n, v.block_stride))
         assert np.array_equal(norms.download(np.float64, 12), want.download(np.float64, 12))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("edge,wg,zchunk", [(32, 256, 8), (32, 512, 16), (32, 256, 32), (16, 128, 8), (16, 128, 16)])
+@pytest.mark.parametrize("walls", ["periodic", "mixed"])
+def test_run_with_a_pinned_block_tile(gpu, dtype, edge, wg, zchunk, walls):
+    """The two-step kernel on block tiles at every pinned z depth: each of ten runs
+    from the same field gives the single steps' field (a workgroup's last plane
+    was stored wrong in some of them)."""
+    nb, n = tuple(np.array((6, 5, 4)) * (32 // edge)), (edge,) * 3
+    lists = [MIXED if walls == "mixed" else []]
+    u, slabs, _ = build(nb, n, dtype, 89, lists)
+    t, _, _ = build(nb, n, dtype, 89, lists)
+    a, _, _ = build(nb, n, dtype, 89, lists)
+    b, _, _ = build(nb, n, dtype, 89, lists)
+    dt = 0.1 / 192 ** 2
+    for k in range(4):
+        cnv.diffusion_step(a, b, dt)
+        a, b = b, a
+    base = cnv.tune_diffusion_run(dtype, edge)
+    try:
+        cnv.set_tune_diffusion_run(dtype, edge, wg, zchunk)
+        for rep in range(10):
+            u.upload(0, slabs[0])
+            assert cnv.diffusion_run(u, t, 4, dt) is u
+            diff = cnv.grid_compare(u, a)
+            assert diff[0] == 0.0 and diff[2] == 0.0, (rep, diff)
+    finally:
+        cnv.set_tune_diffusion_run(dtype, edge, *base)

@@ -655,7 +655,8 @@ def autotune_stencil7(u, out, iters=20):
 
 def autotune_diffusion_run(u, tmp, iters=20):
     """Pick (workgroup size, z-planes per tile) of the two-step kernel that
-    diffusion_run uses on periodic grids of 16^3 / 32^3 blocks; returns
+    diffusion_run uses on larger grids of 16^3 / 32^3 blocks (on all of them
+    where it is not the built-in tile), on a periodic grid; returns
     (wg, zchunk, table).  tmp is overwritten."""
     wg, zc, nr = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     res = np.zeros(3 * 64, dtype=np.float64)

@@ -211,18 +211,22 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
         hc[h] = sx.cst || sy.cst;
     }
     // WALL: ring cells past a wall: a constant (1), or written by the thread
-    // of the cell next to it (2); the factors of this thread's cells next to
-    // a mirror or edge wall (0: none) and of the z walls
+    // of the cell next to it (2); whether this thread's cells lie next to a
+    // mirror or edge wall, and its factor (a Symmetry factor may be 0 in T)
     int rk[RS];
     T rv[RS];
-    T gx0 = (T)0, gx1 = (T)0, gy0 = (T)0, gy1 = (T)0, gz0 = (T)0, gz1 = (T)0;
+    struct Ghost {
+        bool on;
+        T f;
+    };
+    Ghost gx0{}, gx1{}, gy0{}, gy1{}, gz0{}, gz1{};
     if constexpr (WALL) {
         auto past = [&](int d, int side, int b, int nb) { // rule past this side of the block, 0: a neighbour
             return (side ? b == nb - 1 : b == 0) ? fc.fm[d][side] : FM_PERIODIC;
         };
-        auto factor = [&](int d, int side, int b, int nb) -> T {
+        auto factor = [&](int d, int side, int b, int nb) -> Ghost {
             const int k = past(d, side, b, nb);
-            return k == FM_MIRROR ? (T)fc.fv[d][side] : k == FM_EDGE ? (T)1 : (T)0;
+            return {k == FM_MIRROR || k == FM_EDGE, k == FM_MIRROR ? (T)fc.fv[d][side] : (T)1};
         };
         if (x0 == 0)
             gx0 = factor(0, 0, bx, nbx);
@@ -389,15 +393,15 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
             if (inner) {
                 *reinterpret_cast<V *>(Bq + (y + 1) * PA + VEC + x0) = res;
                 if constexpr (WALL) { // ghosts of u^{n+1} past mirror and edge walls
-                    if (gx0 != (T)0)
-                        Bq[(y + 1) * PA + VEC - 1] = gx0 * res.v[0];
-                    if (gx1 != (T)0)
-                        Bq[(y + 1) * PA + VEC + N] = gx1 * res.v[VEC - 1];
-                    if ((y == 0 && gy0 != (T)0) || (y == N - 1 && gy1 != (T)0)) {
+                    if (gx0.on)
+                        Bq[(y + 1) * PA + VEC - 1] = gx0.f * res.v[0];
+                    if (gx1.on)
+                        Bq[(y + 1) * PA + VEC + N] = gx1.f * res.v[VEC - 1];
+                    if ((y == 0 && gy0.on) || (y == N - 1 && gy1.on)) {
                         V g;
 #pragma unroll
                         for (int v = 0; v < VEC; ++v)
-                            g.v[v] = (y == 0 ? gy0 : gy1) * res.v[v];
+                            g.v[v] = (y == 0 ? gy0.f : gy1.f) * res.v[v];
                         *reinterpret_cast<V *>(Bq + (y == 0 ? 0 : N + 1) * PA + VEC + x0) = g;
                     }
                 }
@@ -470,10 +474,10 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
                     const T xp = v == VEC - 1 ? xr : c1[r].v[v + 1];
                     T zm = m1[r].v[v], zp = n1[r].v[v];
                     if constexpr (WALL) {
-                        if (q - 1 == 0 && gz0 != (T)0)
-                            zm = gz0 * c1[r].v[v];
-                        if (q - 1 == N - 1 && gz1 != (T)0)
-                            zp = gz1 * c1[r].v[v];
+                        if (q - 1 == 0 && gz0.on)
+                            zm = gz0.f * c1[r].v[v];
+                        if (q - 1 == N - 1 && gz1.on)
+                            zp = gz1.f * c1[r].v[v];
                     }
                     res.v[v] = euler(c1[r].v[v], xm, xp, ym.v[v], yp.v[v], zm, zp);
                     acc1 = __builtin_fma((double)c1[r].v[v], (double)c1[r].v[v], acc1);

@@ -627,17 +627,23 @@ static int launch_generic(cnv_batch_s *b, hipStream_t st)
 // Planes per item of the single launch for a grid: the tuned depth of its
 // (block edge, ghost width), else by its operator.  A WENO5 item marches its
 // planes at about 2 us each, so a 32-plane item is 75 us of one workgroup: the
-// launch's tail, and all of a small batch.  WENO5 takes 8 planes (16 when the
-// batch holds 1024 32^3 blocks of it: the four extra planes a chunk reads then
-// cost more than the tail), diffusion whole blocks, other shapes 8 planes.  Us
-// per step with 32 / 16 / 8 WENO5 planes: 96 grids (2333 32^3 blocks of WENO5)
+// launch's tail, and all of a small batch.  WENO5 and 16^3 blocks take 8 planes
+// (16 when the batch holds 1024 32^3 blocks of WENO5: the planes that chunks read
+// twice then cost more than the tail), diffusion on 32^3 blocks whole blocks.
+// Us per step with 32 / 16 / 8 WENO5 planes: 96 grids (2333 32^3 blocks of WENO5)
 // 716 / 683 / 693, 35 grids (354 blocks) 187 / 150 / 129, 35 small grids 78 / 43 /
-// 31; diffusion items of 8 planes instead of 32: 129 -> 140 and no gain elsewhere.
+// 31; diffusion on 32^3 with 8 planes instead of 32: 129 -> 140 and no gain
+// elsewhere; 12 grids of 16^3 diffusion with 16 / 8 planes 14.9 / 9.7, the 96 grids
+// 641 / 673 (both operators on 16^3).  Other shapes take up to 32 or 8 planes by
+// their edge, halved until the tile fits: 12 grids of WENO5 on 32x32x20 blocks 65
+// with the 5 planes of that, 118 with 8, whose 62 KB leave two workgroups per CU.
 static int one_zdepth(const cnv_batch_s *b, const cnv_batch_item &it)
 {
     const cnv_grid_s *g = it.in;
     const std::pair<int, int> key(class_key_edge(g), it.ghost);
-    int nz = !marchable(it) ? 8 : it.op == CNV_OP_DIFFUSION ? 32 : b->one_deep ? 16 : 8;
+    int nz = key.first >= 32 ? 32 : 8;
+    if (marchable(it) && (it.op == CNV_OP_WENO5 || key.first == 16))
+        nz = b->one_deep ? 16 : 8;
     if (b->zmap.count(key))
         nz = b->zmap.at(key);
     return std::max(1, std::min(nz, g->desc.block_cells[2]));

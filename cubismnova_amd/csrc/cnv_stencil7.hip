@@ -338,16 +338,26 @@ static void launch_cols(const S7Args &a, const ColShape &s, unsigned nwg, bool b
         hipLaunchKernelGGL((k_stencil7_cols<T, VEC, MODE, SUMSQ, false>), dim3(nwg), dim3(kColWG), 0, st, a, s);
 }
 
+// The sizes the column kernel takes: gx groups of 256 cells per block, gy blocks
+// of all components.
+static int check_cols(const Geom &G, int ncomp, long long *gx, long long *gy)
+{
+    *gx = ((long long)G.n[0] * G.n[1] * G.n[2] + 255) / 256;
+    *gy = (long long)G.nb[0] * G.nb[1] * G.nb[2] * ncomp;
+    if (*gy > 65535 || *gx > 65535)
+        return fail(CNV_ERR_UNSUPPORTED, "grid too large for the generic stencil kernel");
+    return CNV_OK;
+}
+
 // The column kernel on blocks of any shape.
 template <typename T, int MODE, bool SUMSQ>
 static int run_cols(S7Args &a, int ncomp, hipStream_t st, bool finalize, int *nparts, long long cap)
 {
     const int *n = a.G.n;
-    const long long cells = (long long)n[0] * n[1] * n[2];
-    const long long gx = (cells + 255) / 256;
-    const long long gy = (long long)a.G.nb[0] * a.G.nb[1] * a.G.nb[2] * ncomp;
-    if (gy > 65535 || gx > 65535)
-        return fail(CNV_ERR_UNSUPPORTED, "grid too large for the generic stencil kernel");
+    long long gx = 0, gy = 0;
+    const int rc = check_cols(a.G, ncomp, &gx, &gy);
+    if (rc != CNV_OK)
+        return rc;
     if (SUMSQ && cap > 0 && gx * gy > cap)
         return fail(CNV_ERR_SIZE, "grid needs more norm partials than the scratch array holds");
     const int vec = col_vec(n[0], sizeof(T));
@@ -389,6 +399,8 @@ static bool cols_for_small(const Geom &G, int ncomp, size_t elem)
     return cells * (long long)elem < 40ll * 1000 * 1000;
 }
 
+static bool march_edge(const int n[3]) { return n[0] == n[1] && (n[0] == 16 || n[0] == 32 || n[0] == 64); }
+
 // cap: partials the buffer at a.partials holds (0: sized by the caller for
 // the largest launch)
 template <typename T, int MODE, bool SUMSQ>
@@ -397,8 +409,7 @@ static int run_t(S7Args &a, int ncomp, hipStream_t st, int force_generic, const 
 {
     const int *n = a.G.n;
     const long long nbt = (long long)a.G.nb[0] * a.G.nb[1] * a.G.nb[2];
-    const bool cubic_xy = n[0] == n[1];
-    if (!force_generic && cubic_xy && (n[0] == 16 || n[0] == 32 || n[0] == 64)) {
+    if (!force_generic && march_edge(n)) {
         bool pinned = false;
         S7Tune tu = over ? *over : s7_default_tune(sizeof(T) == 8 ? CNV_F64 : CNV_F32, n[0], &pinned);
         if (!over && !pinned && cols_for_small(a.G, ncomp, sizeof(T)))
@@ -450,6 +461,30 @@ static int check_faces(cnv_grid_s *g, int comp)
     return CNV_OK;
 }
 
+// What a single step refuses on a grid, before any launch.
+static int check_components(const cnv_grid_s *u, int ncomp)
+{
+    if (ncomp > kMaxComp)
+        return fail(CNV_ERR_UNSUPPORTED, "more than 8 components in one stencil call");
+    for (int d = 0; d < 3; ++d)
+        if (u->desc.block_cells[d] < 1)
+            return fail(CNV_ERR_INVALID, "empty block");
+    return CNV_OK;
+}
+
+static int check_step(cnv_grid_s *u)
+{
+    int rc = check_components(u, u->desc.ncomp);
+    for (int c = 0; rc == CNV_OK && c < u->desc.ncomp; ++c) {
+        std::lock_guard<std::mutex> lk(u->mtx);
+        rc = check_faces(u, c);
+    }
+    long long gx, gy;
+    if (rc == CNV_OK && (force_generic() || !march_edge(u->desc.block_cells)))
+        rc = check_cols(geom_of(u), u->desc.ncomp, &gx, &gy);
+    return rc;
+}
+
 // State of one launch inside a multi-step run (cnv_diffusion_run).
 struct S7Run {
     double *partials;          // this launch's partial buffer
@@ -470,11 +505,9 @@ static int launch_stencil7_t(cnv_grid_s *u, cnv_grid_s *out, cnv_grid_s *lap, in
                              int ncomp, int mode, double nu_dt, double *sumsq, hipStream_t st,
                              const S7Tune *over, const S7Run *run = nullptr, const S7Scratch *scr = nullptr)
 {
-    if (ncomp > kMaxComp)
-        return fail(CNV_ERR_UNSUPPORTED, "more than 8 components in one stencil call");
-    for (int d = 0; d < 3; ++d)
-        if (u->desc.block_cells[d] < 1)
-            return fail(CNV_ERR_INVALID, "empty block");
+    const int bad = check_components(u, ncomp);
+    if (bad != CNV_OK)
+        return bad;
     S7Args a;
     a.u = static_cast<const char *>(u->data);
     a.out = static_cast<char *>(out->data);
@@ -992,10 +1025,20 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
     int rz = 0, nt2 = 0;
     X2Faces faces[kX2MaxComp];
     bool periodic = false, walls = false;
-    if (nsteps >= 4 && !force_generic()) {
+    if (nsteps >= 4 && !force_generic())
         periodic = run_periodic(u) && run_periodic(tmp);
-        walls = !periodic && run_walls(u, faces);
+    // A run is refused before its first launch or not at all: it ends in single
+    // steps unless all of them pair up, and the launches of several steps take
+    // grids (components, blocks, list lengths) that a single step does not.
+    // Periodic grids of 16^3 and 32^3 blocks step in pairs whatever a single
+    // step takes.
+    if (nsteps > 0 && !(periodic && x2_shape_ok(u) && nsteps % 4 == 0)) {
+        const int rc = check_step(u);
+        if (rc != CNV_OK)
+            return rc;
     }
+    if (nsteps >= 4 && !force_generic())
+        walls = !periodic && run_walls(u, faces);
     if (periodic || walls) {
         const bool shape = x2_shape_ok(u), pinned = shape && x2_tile(u, &xwg, &xz);
         // the block-marching kernel, whose halo is the cheaper one, but for FP32 on

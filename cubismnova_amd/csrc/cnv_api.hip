@@ -41,6 +41,43 @@ int check_stencil(const cnv_stencil *s)
     return CNV_OK;
 }
 
+FaceRules face_rules(const FaceInfo &f)
+{
+    FaceRules r{};
+    for (int k = 0; k < 6; ++k) {
+        const int d = k >> 1, s = k & 1;
+        r.fm[k] = f.uniform ? f.fm[d][s] : FM_CONST;
+        r.v[k] = f.uniform ? f.fv[d][s] : std::nan("");
+    }
+    return r;
+}
+
+int ensure_rules(cnv_grid_s *g, const hipStream_t *run)
+{
+    if (g->rules_version == g->bc_version)
+        return CNV_OK;
+    const bool first = g->rules_version == ~0ull;
+    g->rules_host.resize((size_t)g->nslabs);
+    for (int c = 0; c < g->nslabs; ++c) {
+        // cleared lists leave the rules, like the table, to what was recorded with them
+        const FaceInfo &f = face_info(g, c);
+        if (first || f.longest > 0)
+            g->rules_host[c] = face_rules(f);
+    }
+    if (!first) // kernels still queued on any stream may read them
+        CNV_HIP(hipDeviceSynchronize());
+    if (run && g->nslabs <= kX2MaxComp) { // (a copy is 20 us of the first run on a grid, this 4)
+        const int rc = launch_rules(g, *run);
+        if (rc != CNV_OK)
+            return rc;
+    } else {
+        CNV_HIP(hipMemcpy(g->rules, g->rules_host.data(), sizeof(FaceRules) * (size_t)g->nslabs,
+                          hipMemcpyHostToDevice));
+    }
+    g->rules_version = g->bc_version;
+    return CNV_OK;
+}
+
 int ensure_bc_table(cnv_grid_s *g, int comp)
 {
     BCTable &t = g->tables[comp];
@@ -94,7 +131,7 @@ int ensure_bc_table(cnv_grid_s *g, int comp)
     CNV_HIP(hipMemcpy(t.heads, image.get(), hb + eb, hipMemcpyHostToDevice));
     t.any = ne > 0;
     t.version = g->bc_version;
-    return CNV_OK;
+    return g->rules_version == ~0ull ? CNV_OK : ensure_rules(g, nullptr); // both or none follow the lists
 }
 
 // Every block's BC list resolved for a stencil that reads both sides (-1, 2)
@@ -164,10 +201,15 @@ const FaceInfo &face_info(cnv_grid_s *g, int comp)
 int ensure_partials(cnv_grid_s *g, size_t n)
 {
     if (n > g->partials_cap) {
-        if (g->partials)
-            CNV_HIP(hipFree(g->partials));
+        if (g->rules)
+            CNV_HIP(hipFree(g->rules));
+        g->rules = nullptr;
         g->partials = nullptr;
-        CNV_HIP(hipMalloc((void **)&g->partials, 2 * sizeof(double) * n));
+        g->partials_cap = 0;
+        const size_t rb = sizeof(FaceRules) * (size_t)g->nslabs;
+        CNV_HIP(hipMalloc((void **)&g->rules, rb + 2 * sizeof(double) * n));
+        g->rules_version = ~0ull;
+        g->partials = reinterpret_cast<double *>(reinterpret_cast<char *>(g->rules) + rb);
         g->partials_cap = n;
     }
     return CNV_OK;
@@ -416,13 +458,15 @@ static int grid_make(const cnv_grid_desc *desc, void *data, size_t data_bytes, c
     // reduction scratch sized for the largest launch of any operator, so that
     // no call allocates later (calls may be recorded into a HIP graph)
     const size_t nparts = (size_t)nbt * desc->ncomp * ((size_t)(cells + 255) / 256 + desc->block_cells[2]) + 4096;
-    const hipError_t e = hipMalloc((void **)&g->partials, 2 * sizeof(double) * nparts); // two halves
+    const size_t rb = sizeof(FaceRules) * (size_t)nslabs;
+    const hipError_t e = hipMalloc((void **)&g->rules, rb + 2 * sizeof(double) * nparts); // two halves
     if (e != hipSuccess) {
         if (g->owns_data)
             (void)hipFree(g->data);
         delete g;
         return fail(CNV_ERR_ALLOC, std::string("scratch allocation: ") + hipGetErrorString(e));
     }
+    g->partials = reinterpret_cast<double *>(reinterpret_cast<char *>(g->rules) + rb);
     g->partials_cap = nparts;
     *out = g;
     return CNV_OK;
@@ -454,8 +498,8 @@ int cnv_grid_destroy(cnv_grid g)
         if (t.heads)
             (void)hipFree(t.heads);
     }
-    if (g->partials)
-        (void)hipFree(g->partials);
+    if (g->rules)
+        (void)hipFree(g->rules);
     if (g->czm_dev)
         (void)hipFree(g->czm_dev);
     if (g->czp_dev)
@@ -1150,6 +1194,10 @@ int cnv_grid_prepare(cnv_grid g)
             std::lock_guard<std::mutex> lk(g->mtx);
             CNV_CHECK(ensure_bc_table(g, c));
         }
+    }
+    if (g->desc.entity == CNV_CELL && g->bc_version > 0) {
+        std::lock_guard<std::mutex> lk(g->mtx);
+        CNV_CHECK(ensure_rules(g, nullptr));
     }
     return CNV_OK;
     CNV_GUARD_END

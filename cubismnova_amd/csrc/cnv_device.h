@@ -176,6 +176,21 @@ __device__ inline T face_val(const FaceSrc<T> &f, long long i)
     return f.mode == 1 ? f.s * v : v;
 }
 
+// Rules in the grid's memory or in the kernel's arguments: memory that no kernel
+// writes, so constant to the compiler, which reads the rule of a face that is
+// uniform in a wave by scalar loads.
+typedef const __attribute__((address_space(4))) FaceRules *DevRules;
+
+// Rules of component comp, by value (VAL) or as p says; `at`: offset of r in the
+// kernel's one argument.
+template <bool VAL = false>
+__device__ inline DevRules rules_of(const RunRules &r, size_t at, int comp)
+{
+    typedef const __attribute__((address_space(4))) char *Bytes;
+    const FaceRules *p = VAL ? nullptr : r.p[comp];
+    return p ? (DevRules)p : (DevRules)((Bytes)__builtin_amdgcn_kernarg_segment_ptr() + at) + comp;
+}
+
 // Resolve the six one-layer faces of block `blk` (ghost layer 1 of the lab,
 // the only one the 7-point operators read; the same for any ghost width).
 template <typename T>

@@ -82,6 +82,13 @@ struct FaceInfo {
     double fv[3][2] = {};
 };
 
+// The same for kernels: FM_* of the face 2 dir + side and its constant or sign.
+// Lists that give some face more than one rule are written as constants of NaN.
+struct FaceRules {
+    int fm[6];
+    double v[6];
+};
+
 struct BCTable {
     FaceInfo faces;
     uint64_t version = ~0ull; // BC version this table was built from
@@ -112,6 +119,11 @@ struct cnv_grid_s {
     // scratch for deterministic reductions: per-tile partial sums, two halves
     // of partials_cap doubles each
     double *partials = nullptr;
+    // rules of every component in the same allocation, before the partials, and
+    // the BC version they were written for (~0: never)
+    cnv::FaceRules *rules = nullptr;
+    std::vector<cnv::FaceRules> rules_host;
+    uint64_t rules_version = ~0ull;
 
     // z metric of a stretched mesh (per global z cell), set on first use
     double *czm_dev = nullptr;
@@ -176,6 +188,10 @@ int ensure_bc_table(cnv_grid_s *g, int comp);
 // The faces of component comp, derived again when its BC lists changed; the
 // caller holds the grid's mutex.
 const FaceInfo &face_info(cnv_grid_s *g, int comp);
+// Write the rules of every component to the device (if stale): before the next
+// launch on `run`'s stream, or at once where it is null.
+int ensure_rules(cnv_grid_s *g, const hipStream_t *run);
+int launch_rules(cnv_grid_s *g, hipStream_t st);
 // Make sure the reduction scratch holds at least n partials.
 int ensure_partials(cnv_grid_s *g, size_t n);
 
@@ -254,15 +270,21 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
 // all its blocks and every inner face is a neighbour copy (cnv_jacobi2.hip)
 bool jacobi2_faces(cnv_grid_s *g, int comp, int fm[3][2], double fv[3][2]);
 
-// two Euler steps per launch on periodic grids, and on grids with walls with
-// the faces of every component (cnv_stencil7x2.hip)
+// two Euler steps per launch on periodic grids, and on grids with walls by the
+// rules of every component (cnv_stencil7x2.hip)
 constexpr int kX2MaxComp = 8;
-struct X2Faces {
-    int fm[3][2];
-    double fv[3][2];
+// The rules of every component for the launches that take several steps between
+// walls.  A recorded launch reads those of components with lists from the
+// grid's memory (p), so that replays follow changed lists as those of single
+// steps do; others (p null) carry them.
+struct RunRules {
+    FaceRules val[kX2MaxComp];
+    const FaceRules *p[kX2MaxComp];
 };
 
-bool run_walls(cnv_grid_s *u, X2Faces *faces);
+FaceRules face_rules(const FaceInfo &f);
+bool run_walls(cnv_grid_s *u);
+int run_rules(cnv_grid_s *g, int ncomp, hipStream_t st, RunRules &r);
 bool run_periodic(cnv_grid_s *u);
 bool x2_shape_ok(const cnv_grid_s *u);
 bool x2_applicable(cnv_grid_s *u);
@@ -270,14 +292,14 @@ long long x2_tiles(const cnv_grid_s *u, int zchunk);
 bool x2_tile(cnv_grid_s *u, int *wg, int *zchunk);
 int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, double nu_dt, double *part1, double *part2,
                         const double *const prev_p[2], const int prev_n[2], double *const prev_out[2], int wg,
-                        int zchunk, int *nparts, hipStream_t st, const X2Faces *faces = nullptr);
+                        int zchunk, int *nparts, hipStream_t st, const RunRules *rules = nullptr);
 // 2 or 4 Euler steps or Jacobi sweeps per launch on LDS tiles of the domain, any
 // block shape (cnv_tile.hip): tiles of a launch, the steps a grid takes (0:
 // another kernel), the launches; the launches of n steps, up to k at a time
 int tile_count(const cnv_grid_s *u, int k, int ncomp);
 int tile_steps(const cnv_grid_s *u, bool block_tiles, bool walls);
 int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int k, double nu_dt, double *part, const double *prev_p,
-                      int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st);
+                      int nprev, int prev_n, double *prev_out, const RunRules *rules, hipStream_t st);
 int launch_tile_jacobi(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s *out, int co, int k, double omega,
                        hipStream_t st);
 std::vector<int> run_launches(int n, int k);
@@ -285,7 +307,7 @@ std::vector<int> run_launches(int n, int k);
 // shape (cnv_run2.hip): tiles (0: not available) and planes per tile; the launch
 int run2_tiles(const cnv_grid_s *u, int *zchunk);
 int launch_run2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int zchunk, double nu_dt, double *part, const double *prev_p,
-                int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st);
+                int nprev, int prev_n, double *prev_out, const RunRules *rules, hipStream_t st);
 int x2_set_tune(int dtype, int edge, int wg, int zchunk);
 int x2_get_tune(int dtype, int edge, int *wg, int *zchunk);
 int autotune_x2(cnv_grid_s *u, cnv_grid_s *out, int iters, int *best_wg, int *best_z, double *results,

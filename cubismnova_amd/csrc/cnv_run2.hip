@@ -38,7 +38,7 @@ struct Run2Args {
     int nb[3], n[3], ng[3], nt[3];
     FastDiv dn[3];
     int zchunk, ntiles; // ntiles: of all components
-    X2Faces faces[kX2MaxComp];
+    RunRules rules;
     double ih2[3], nudt;
     double *part; // norms: part[j * ntiles + tile]
     const double *prev_p;
@@ -97,12 +97,12 @@ __global__ __launch_bounds__(kRun2WG) void k_run2(const Run2Args a)
     const int gx = tx * CX + (q - 1) * VEC, gy = ty * CY + r - 2;
     const char *ub = a.u + (long long)comp * a.cs_u;
     char *ob = a.out + (long long)comp * a.cs_o;
-    const X2Faces &fc = a.faces[WALL ? comp : 0];
+    const DevRules rules = rules_of(a.rules, offsetof(Run2Args, rules), WALL ? comp : 0);
 
     // cell index inside the domain: periodic axes wrapped, walls clamped
     // (cells past a wall are loaded and never used)
     auto inside = [&](int g, int d, int n, int last) {
-        if (!WALL || fc.fm[d][0] == FM_PERIODIC) {
+        if (!WALL || rules->fm[2 * d] == FM_PERIODIC) {
             g %= n;
             return g < 0 ? g + n : g;
         }
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kRun2WG) void k_run2(const Run2Args a)
         ++p.z;
         return p;
     };
-    const bool pz = !WALL || fc.fm[2][0] == FM_PERIODIC;
+    const bool pz = !WALL || rules->fm[4] == FM_PERIODIC;
     Plane in = plane(inside(Z0 - 2, 2, NZ, NZ - 1)), out = plane(Z0);
     int zin = Z0 - 2; // plane of the next load; `in` is it wrapped or clamped
     auto load = [&]() __attribute__((always_inline)) {
@@ -166,15 +166,15 @@ __global__ __launch_bounds__(kRun2WG) void k_run2(const Run2Args a)
     const int lo = ((r + 1) * LR + q) * VEC;
     const T ihx2 = (T)a.ih2[0], ihy2 = (T)a.ih2[1], ihz2 = (T)a.ih2[2], nudt = (T)a.nudt;
     // walls next to the lane's cells; the w* flags are uniform in a wave
-    const bool xlo = WALL && fc.fm[0][0] != FM_PERIODIC && gx == 0;
-    const int xhi = WALL && fc.fm[0][1] != FM_PERIODIC ? NX - 1 - gx : -1; // element next to the upper wall
-    const bool ylo = WALL && fc.fm[1][0] != FM_PERIODIC && gy == 0;
-    const bool yhi = WALL && fc.fm[1][1] != FM_PERIODIC && gy == NY - 1;
+    const bool xlo = WALL && rules->fm[0] != FM_PERIODIC && gx == 0;
+    const int xhi = WALL && rules->fm[1] != FM_PERIODIC ? NX - 1 - gx : -1; // element next to the upper wall
+    const bool ylo = WALL && rules->fm[2] != FM_PERIODIC && gy == 0;
+    const bool yhi = WALL && rules->fm[3] != FM_PERIODIC && gy == NY - 1;
     const bool wx = WALL && __builtin_amdgcn_ballot_w64(xlo || (xhi >= 0 && xhi < VEC)) != 0;
     const bool wy = WALL && __builtin_amdgcn_ballot_w64(ylo || yhi) != 0;
     auto wall = [&](int d, int side, T v) __attribute__((always_inline)) {
-        return fc.fm[d][side] == FM_CONST ? (T)fc.fv[d][side]
-               : fc.fm[d][side] == FM_MIRROR ? (T)fc.fv[d][side] * v : v;
+        const int k = rules->fm[2 * d + side];
+        return k == FM_CONST ? (T)rules->v[2 * d + side] : k == FM_MIRROR ? (T)rules->v[2 * d + side] * v : v;
     };
     // one step of plane z from its own and the neighbouring planes, in the
     // single step's order
@@ -201,11 +201,11 @@ __global__ __launch_bounds__(kRun2WG) void k_run2(const Run2Args a)
                     yp.v[v] = yhi ? wall(1, 1, c.v[v]) : yp.v[v];
                 }
             }
-            if (z == 0 && fc.fm[2][0] != FM_PERIODIC)
+            if (z == 0 && rules->fm[4] != FM_PERIODIC)
 #pragma unroll
                 for (int v = 0; v < VEC; ++v)
                     zm.v[v] = wall(2, 0, c.v[v]);
-            if (z == NZ - 1 && fc.fm[2][1] != FM_PERIODIC)
+            if (z == NZ - 1 && rules->fm[5] != FM_PERIODIC)
 #pragma unroll
                 for (int v = 0; v < VEC; ++v)
                     zp.v[v] = wall(2, 1, c.v[v]);
@@ -391,7 +391,7 @@ int run2_tiles(const cnv_grid_s *u, int *zchunk)
 }
 
 int launch_run2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int zchunk, double nu_dt, double *part, const double *prev_p,
-                int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st)
+                int nprev, int prev_n, double *prev_out, const RunRules *rules, hipStream_t st)
 {
     Run2Args a{};
     const bool f64 = u->desc.dtype == CNV_F64;
@@ -401,8 +401,8 @@ int launch_run2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int zchunk, double nu
     a.out = static_cast<char *>(out->data);
     a.cs_u = (long long)u->component_bytes;
     a.cs_o = (long long)out->component_bytes;
-    for (int c = 0; faces && c < ncomp; ++c)
-        a.faces[c] = faces[c];
+    if (rules)
+        a.rules = *rules;
     for (int d = 0; d < 3; ++d)
         a.ih2[d] = 1. / (u->h[d] * u->h[d]);
     a.nudt = nu_dt;
@@ -411,7 +411,7 @@ int launch_run2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int zchunk, double nu
     a.nprev = nprev;
     a.prev_n = prev_n;
     a.prev_out = prev_out;
-    const bool wall = faces != nullptr, vec = u->desc.block_cells[0] % (f64 ? 2 : 4) == 0;
+    const bool wall = rules != nullptr, vec = u->desc.block_cells[0] % (f64 ? 2 : 4) == 0;
     if (f64)
         vec ? run2_launch<double, true>(a, wall, st) : run2_launch<double, false>(a, wall, st);
     else

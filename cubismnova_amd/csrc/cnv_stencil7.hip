@@ -1023,22 +1023,21 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
     int xwg = 0, xz = 0, k = 1;
     bool tiles = false;
     int rz = 0, nt2 = 0;
-    X2Faces faces[kX2MaxComp];
     bool periodic = false, walls = false;
     if (nsteps >= 4 && !force_generic())
-        periodic = run_periodic(u) && run_periodic(tmp);
+        periodic = run_periodic(u);
     // A run is refused before its first launch or not at all: it ends in single
     // steps unless all of them pair up, and the launches of several steps take
     // grids (components, blocks, list lengths) that a single step does not.
     // Periodic grids of 16^3 and 32^3 blocks step in pairs whatever a single
     // step takes.
-    if (nsteps > 0 && !(periodic && x2_shape_ok(u) && nsteps % 4 == 0)) {
+    if (nsteps > 0 && !(periodic && run_periodic(tmp) && x2_shape_ok(u) && nsteps % 4 == 0)) {
         const int rc = check_step(u);
         if (rc != CNV_OK)
             return rc;
     }
     if (nsteps >= 4 && !force_generic())
-        walls = !periodic && run_walls(u, faces);
+        walls = !periodic && run_walls(u);
     if (periodic || walls) {
         const bool shape = x2_shape_ok(u), pinned = shape && x2_tile(u, &xwg, &xz);
         // the block-marching kernel, whose halo is the cheaper one, but for FP32 on
@@ -1057,6 +1056,12 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
             k = nt2 > 0 && (size_t)2 * nt2 <= cap ? 2 : 1;
         }
     }
+    RunRules rules[2] = {}; // of u and of tmp
+    for (int g = 0; walls && k > 1 && g < 2; ++g) {
+        const int rc = run_rules(g == 0 ? u : tmp, nc, st, rules[g]);
+        if (rc != CNV_OK)
+            return rc;
+    }
     const double *prev = nullptr; // nprev sets of prev_n partials, consecutive
     int nprev = 0, prev_n = 0;
     double *prev_out = nullptr;
@@ -1072,12 +1077,13 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
     for (const int kk : run_launches(nsteps, k)) {
         cnv_grid_s *a = L % 2 == 0 ? u : tmp, *b = L % 2 == 0 ? tmp : u;
         double *part = norms ? P[L % 2] : nullptr;
+        const RunRules *wr = walls ? &rules[L % 2] : nullptr;
         int nt = 0, rc = CNV_OK;
         if (kk > 1 && tiles) {
-            rc = launch_tile_euler(a, b, nc, kk, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
+            rc = launch_tile_euler(a, b, nc, kk, nu_dt, part, prev, nprev, prev_n, prev_out, wr, st);
             nt = tile_count(u, kk, nc);
         } else if (kk > 1 && nt2 > 0) {
-            rc = launch_run2(a, b, nc, rz, nu_dt, part, prev, nprev, prev_n, prev_out, walls ? faces : nullptr, st);
+            rc = launch_run2(a, b, nc, rz, nu_dt, part, prev, nprev, prev_n, prev_out, wr, st);
             nt = nt2;
         } else {
             if (nprev > 2)
@@ -1087,7 +1093,7 @@ int launch_diffusion_run(cnv_grid_s *u, cnv_grid_s *tmp, int nsteps, double nu_d
             double *po[2] = {prev_out, prev_out + 1};
             if (rc == CNV_OK && kk > 1) {
                 rc = launch_diffusion_x2(a, b, nc, nu_dt, part, part ? part + x2_tiles(u, xz) : nullptr, pp, pn, po,
-                                         xwg, xz, &nt, st, walls ? faces : nullptr);
+                                         xwg, xz, &nt, st, wr);
             } else if (rc == CNV_OK) {
                 S7Run run;
                 run.partials = part;

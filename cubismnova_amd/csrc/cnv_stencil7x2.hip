@@ -35,7 +35,7 @@ struct X2Args {
     const double *prev_p[2];
     int prev_n[2];
     double *prev_out[2];
-    X2Faces faces[kX2MaxComp]; // WALL kernels only
+    RunRules rules; // WALL kernels only
 };
 
 template <typename T, int N, int WG>
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
     // WALL: the value read, times hm, or the constant hv past a Dirichlet wall
     T hm[HS], hv[HS];
     bool hc[HS];
-    const X2Faces &fc = a.faces[WALL ? comp : 0];
+    const DevRules rules = rules_of(a.rules, offsetof(X2Args, rules), WALL ? comp : 0);
     // cell l of block b along axis d (l = -2 .. N + 1) as (block, cell) of the
     // source; past a wall the cell next to it and the wall's rule
     struct Src {
@@ -168,13 +168,13 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
         Src r{b, l, (T)1, (T)0, false};
         if (l >= 0 && l < N)
             return r;
-        const int rule = WALL && (side ? b == nb - 1 : b == 0) ? fc.fm[d][side] : FM_PERIODIC;
+        const int rule = WALL && (side ? b == nb - 1 : b == 0) ? rules->fm[2 * d + side] : FM_PERIODIC;
         if (rule == FM_PERIODIC) {
             r.b = wrap(b + (side ? 1 : -1), nb);
             r.l = side ? l - N : l + N;
             return r;
         }
-        const T f = (T)fc.fv[d][side];
+        const T f = (T)rules->v[2 * d + side];
         r.l = side ? N - 1 : 0;
         r.cst = rule == FM_CONST;
         r.v = f;
@@ -222,11 +222,11 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
     Ghost gx0{}, gx1{}, gy0{}, gy1{}, gz0{}, gz1{};
     if constexpr (WALL) {
         auto past = [&](int d, int side, int b, int nb) { // rule past this side of the block, 0: a neighbour
-            return (side ? b == nb - 1 : b == 0) ? fc.fm[d][side] : FM_PERIODIC;
+            return (side ? b == nb - 1 : b == 0) ? rules->fm[2 * d + side] : FM_PERIODIC;
         };
         auto factor = [&](int d, int side, int b, int nb) -> Ghost {
             const int k = past(d, side, b, nb);
-            return {k == FM_MIRROR || k == FM_EDGE, k == FM_MIRROR ? (T)fc.fv[d][side] : (T)1};
+            return {k == FM_MIRROR || k == FM_EDGE, k == FM_MIRROR ? (T)rules->v[2 * d + side] : (T)1};
         };
         if (x0 == 0)
             gx0 = factor(0, 0, bx, nbx);
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
             const int d = s < 2 * N ? 0 : 1, side = (s / N) & 1;
             const int k = d == 0 ? past(0, side, bx, nbx) : past(1, side, by, nby);
             rk[h] = k == FM_PERIODIC ? 0 : k == FM_CONST ? 1 : 2;
-            rv[h] = (T)fc.fv[d][side];
+            rv[h] = (T)rules->v[2 * d + side];
         }
     }
     const int own = x0 + N * ty; // this thread's first row offset within a plane
@@ -407,10 +407,10 @@ __global__ __launch_bounds__(WG) void k_stencil7x2(const X2Args a)
                 }
             } else if constexpr (WALL) { // a plane past a Dirichlet z wall keeps its constant
                 const int side = q >= N;
-                if ((q < 0 || q >= N) && fc.fm[2][side] == FM_CONST && (side ? bz == nbz - 1 : bz == 0))
+                if ((q < 0 || q >= N) && rules->fm[4 + side] == FM_CONST && (side ? bz == nbz - 1 : bz == 0))
 #pragma unroll
                     for (int v = 0; v < VEC; ++v)
-                        n1[r].v[v] = (T)fc.fv[2][side];
+                        n1[r].v[v] = (T)rules->v[4 + side];
             }
         }
         // plane q - 1 has served: the next u^n plane goes into its slot
@@ -656,24 +656,60 @@ bool x2_shape_ok(const cnv_grid_s *u)
     return n[0] == n[1] && n[1] == n[2] && (n[0] == 16 || n[0] == 32) && u->component_bytes < ((size_t)1 << 31);
 }
 
-// The faces of every component of a grid with walls, each domain face of one
-// rule on all its blocks; false for other grids (they step one at a time).
-bool run_walls(cnv_grid_s *u, X2Faces *faces)
+// Whether each domain face of every component has one rule on all its blocks
+// (other grids with walls step one at a time).
+bool run_walls(cnv_grid_s *u)
 {
     if (u->desc.ncomp > kX2MaxComp)
         return false;
     std::lock_guard<std::mutex> lk(u->mtx);
-    for (int c = 0; c < u->desc.ncomp; ++c) {
-        const FaceInfo &f = face_info(u, c);
-        if (!f.uniform)
+    for (int c = 0; c < u->desc.ncomp; ++c)
+        if (!face_info(u, c).uniform)
             return false;
-        for (int d = 0; d < 3; ++d)
-            for (int s = 0; s < 2; ++s) {
-                faces[c].fm[d][s] = f.fm[d][s];
-                faces[c].fv[d][s] = f.fv[d][s];
-            }
-    }
     return true;
+}
+
+// The rules as an argument, written by one wave.
+struct RulesImage {
+    FaceRules r[kX2MaxComp];
+};
+
+__global__ __launch_bounds__(64) void k_rules(const RulesImage a, FaceRules *out, int n)
+{
+    if ((int)threadIdx.x < n)
+        out[threadIdx.x] = a.r[threadIdx.x];
+}
+
+int launch_rules(cnv_grid_s *g, hipStream_t st)
+{
+    RulesImage a{};
+    for (int c = 0; c < g->nslabs; ++c)
+        a.r[c] = g->rules_host[c];
+    hipLaunchKernelGGL(k_rules, dim3(1), dim3(64), 0, st, a, g->rules, g->nslabs);
+    CNV_HIP(hipGetLastError());
+    return CNV_OK;
+}
+
+// The rules of g's first ncomp components for launches on st that read g.  The
+// device's copies follow the lists in every run, so that a run can be recorded
+// after it was called once, and with them a table that single steps had built.
+int run_rules(cnv_grid_s *g, int ncomp, hipStream_t st, RunRules &r)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (st)
+        (void)hipStreamIsCapturing(st, &cs);
+    std::lock_guard<std::mutex> lk(g->mtx);
+    if (cs != hipStreamCaptureStatusNone && g->rules_version != g->bc_version)
+        return fail(CNV_ERR_INVALID, "BC lists changed since this grid's last run: run once before recording");
+    int rc = ensure_rules(g, &st);
+    for (int c = 0; c < ncomp && rc == CNV_OK; ++c) {
+        const FaceInfo &f = face_info(g, c);
+        r.val[c] = face_rules(f);
+        r.p[c] = cs != hipStreamCaptureStatusNone && f.longest > 0 ? g->rules + c : nullptr;
+        if (g->tables[c].heads)
+            rc = ensure_bc_table(g, c);
+    }
+    return rc;
 }
 
 // No block of the grid carries a BC.
@@ -697,7 +733,7 @@ long long x2_tiles(const cnv_grid_s *u, int zchunk)
 
 int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, double nu_dt, double *part1, double *part2,
                         const double *const prev_p[2], const int prev_n[2], double *const prev_out[2], int wg,
-                        int zchunk, int *nparts, hipStream_t st, const X2Faces *faces)
+                        int zchunk, int *nparts, hipStream_t st, const RunRules *rules)
 {
     const int edge = u->desc.block_cells[0];
     if (wg <= 0 || zchunk <= 0) {
@@ -728,9 +764,9 @@ int launch_diffusion_x2(cnv_grid_s *u, cnv_grid_s *out, int ncomp, double nu_dt,
     const long long ntiles = (long long)a.tiles_per_comp * ncomp;
     if (ntiles >= (1LL << 31))
         return fail(CNV_ERR_UNSUPPORTED, "grid too large for the two-step kernel");
-    for (int c = 0; faces && c < ncomp; ++c)
-        a.faces[c] = faces[c];
-    if (!(faces ? x2_dispatch_wall(u->desc.dtype, edge, zchunk, a, (int)ntiles, st)
+    if (rules)
+        a.rules = *rules;
+    if (!(rules ? x2_dispatch_wall(u->desc.dtype, edge, zchunk, a, (int)ntiles, st)
                 : x2_dispatch(u->desc.dtype, edge, wg, zchunk, a, (int)ntiles, st)))
         return fail(CNV_ERR_UNSUPPORTED, "two-step tile shape not available for this block edge and dtype");
     CNV_HIP(hipGetLastError());

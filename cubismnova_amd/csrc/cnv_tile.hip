@@ -28,7 +28,7 @@ struct TileArgs {
     int nb[3], n[3], ng[3], nt[3];
     FastDiv dn[3];
     int ntiles; // of all components
-    X2Faces faces[kX2MaxComp];
+    RunRules rules;
     double ih2[3], nudt;
     const double *czm, *czp;
     double omega;
@@ -83,7 +83,14 @@ __global__ __launch_bounds__(WG) void k_tile(const TileArgs a)
     const int NX = a.ng[0], NY = a.ng[1], NZ = a.ng[2];
     const T *ub = reinterpret_cast<const T *>(a.u) + (long long)comp * a.cs_u;
     T *ob = reinterpret_cast<T *>(a.out) + (long long)comp * a.cs_o;
-    const X2Faces &fc = a.faces[WALL ? comp : 0];
+    const DevRules rules = rules_of<OP == TILE_JACOBI>(a.rules, offsetof(TileArgs, rules), WALL ? comp : 0);
+    // FM_* of the face 2 dir + side in four bits: the cell loop tests it at every
+    // vector (a 64^3 refined solve 925 us, 980 with a load at each test)
+    unsigned fm = 0u;
+    for (int f = 0; WALL && f < 6; ++f)
+        fm |= (unsigned)rules->fm[f] << (4 * f);
+    auto rule = [&](int d, int side) { return (int)(fm >> (8 * d + 4 * side)) & 15; };
+    auto value = [&](int d, int side) { return (T)rules->v[2 * d + side]; }; // constant or sign of a wall
 
     // element offset of every loaded x, y and z: periodic axes wrapped, walls
     // clamped (those cells are loaded and never used)
@@ -92,7 +99,7 @@ __global__ __launch_bounds__(WG) void k_tile(const TileArgs a)
         const int i = tid - (d == 0 ? 0 : d == 1 ? LX : LX + LY);
         int g = (d == 0 ? X0 - PX : (d == 1 ? Y0 : Z0) - K) + i;
         const int ngd = d == 0 ? NX : d == 1 ? NY : NZ;
-        if (!WALL || fc.fm[d][0] == FM_PERIODIC) {
+        if (!WALL || rule(d, 0) == FM_PERIODIC) {
             g %= ngd;
             g = g < 0 ? g + ngd : g;
         } else {
@@ -178,26 +185,26 @@ __global__ __launch_bounds__(WG) void k_tile(const TileArgs a)
             int xe = -1; // the vector's element next to the upper x wall
             if constexpr (WALL) {
                 auto wall = [&](int d, int side, T v) {
-                    return fc.fm[d][side] == FM_CONST ? (T)fc.fv[d][side]
-                           : fc.fm[d][side] == FM_MIRROR ? (T)fc.fv[d][side] * v : v;
+                    const int k = rule(d, side);
+                    return k == FM_CONST ? value(d, side) : k == FM_MIRROR ? value(d, side) * v : v;
                 };
-                if (gx == 0 && fc.fm[0][0] != FM_PERIODIC)
+                if (gx == 0 && rule(0, 0) != FM_PERIODIC)
                     xl = wall(0, 0, c.v[0]);
-                if (fc.fm[0][1] != FM_PERIODIC)
+                if (rule(0, 1) != FM_PERIODIC)
                     xe = NX - 1 - gx;
-                if (gy == 0 && fc.fm[1][0] != FM_PERIODIC)
+                if (gy == 0 && rule(1, 0) != FM_PERIODIC)
 #pragma unroll
                     for (int v = 0; v < VEC; ++v)
                         ym.v[v] = wall(1, 0, c.v[v]);
-                if (gy == NY - 1 && fc.fm[1][1] != FM_PERIODIC)
+                if (gy == NY - 1 && rule(1, 1) != FM_PERIODIC)
 #pragma unroll
                     for (int v = 0; v < VEC; ++v)
                         yp.v[v] = wall(1, 1, c.v[v]);
-                if (gz == 0 && fc.fm[2][0] != FM_PERIODIC)
+                if (gz == 0 && rule(2, 0) != FM_PERIODIC)
 #pragma unroll
                     for (int v = 0; v < VEC; ++v)
                         zm.v[v] = wall(2, 0, c.v[v]);
-                if (gz == NZ - 1 && fc.fm[2][1] != FM_PERIODIC)
+                if (gz == NZ - 1 && rule(2, 1) != FM_PERIODIC)
 #pragma unroll
                     for (int v = 0; v < VEC; ++v)
                         zp.v[v] = wall(2, 1, c.v[v]);
@@ -217,8 +224,8 @@ __global__ __launch_bounds__(WG) void k_tile(const TileArgs a)
                 const T l = v == 0 ? xl : c.v[v - 1];
                 T h = v == VEC - 1 ? xr : c.v[v + 1];
                 if (WALL && xe == v)
-                    h = fc.fm[0][1] == FM_CONST ? (T)fc.fv[0][1]
-                        : fc.fm[0][1] == FM_MIRROR ? (T)fc.fv[0][1] * e : e;
+                    h = rule(0, 1) == FM_CONST ? value(0, 1)
+                        : rule(0, 1) == FM_MIRROR ? value(0, 1) * e : e;
                 const T ddx = ihx2 * (fms2(e, h) + l);
                 const T ddy = ihy2 * (fms2(e, yp.v[v]) + ym.v[v]);
                 if constexpr (OP == TILE_EULER) {
@@ -386,7 +393,7 @@ int tile_steps(const cnv_grid_s *u, bool block_tiles, bool walls)
 }
 
 int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int k, double nu_dt, double *part, const double *prev_p,
-                      int nprev, int prev_n, double *prev_out, const X2Faces *faces, hipStream_t st)
+                      int nprev, int prev_n, double *prev_out, const RunRules *rules, hipStream_t st)
 {
     TileArgs a{};
     if (!(k == 2 ? tile_layout<2>(u, a, ncomp) : tile_layout<4>(u, a, ncomp)))
@@ -395,11 +402,9 @@ int launch_tile_euler(cnv_grid_s *u, cnv_grid_s *out, int ncomp, int k, double n
     a.out = static_cast<char *>(out->data);
     a.cs_u = (long long)(u->component_bytes / u->elem);
     a.cs_o = (long long)(out->component_bytes / out->elem);
-    bool wall = false;
-    for (int c = 0; faces && c < ncomp; ++c) {
-        a.faces[c] = faces[c];
-        wall = true;
-    }
+    const bool wall = rules != nullptr;
+    if (rules)
+        a.rules = *rules;
     for (int d = 0; d < 3; ++d)
         a.ih2[d] = 1. / (u->h[d] * u->h[d]);
     a.nudt = nu_dt;
@@ -424,11 +429,17 @@ int launch_tile_jacobi(cnv_grid_s *u, int cu, cnv_grid_s *f, int cf, cnv_grid_s 
     TileArgs a{};
     if (!(k == 2 ? u->desc.dtype == CNV_F32 && tile_layout<2>(u, a, 1) : tile_layout<4>(u, a, 1)))
         return fail(CNV_ERR_UNSUPPORTED, "no tile launch of these sweeps on this grid");
-    if (!jacobi2_faces(u, cu, a.faces[0].fm, a.faces[0].fv))
+    int fm[3][2];
+    double fv[3][2];
+    if (!jacobi2_faces(u, cu, fm, fv))
         return fail(CNV_ERR_UNSUPPORTED, "several sweeps per launch need one rule per domain face");
     bool wall = false;
-    for (int d = 0; d < 3; ++d)
-        wall = wall || a.faces[0].fm[d][0] != FM_PERIODIC;
+    for (int f = 0; f < 6; ++f) {
+        const int d = f >> 1, s = f & 1;
+        wall = wall || fm[d][s] != FM_PERIODIC;
+        a.rules.val[0].fm[f] = fm[d][s];
+        a.rules.val[0].v[f] = fv[d][s];
+    }
     a.u = static_cast<const char *>(u->data) + (size_t)cu * u->component_bytes;
     a.f = static_cast<const char *>(f->data) + (size_t)cf * f->component_bytes;
     a.out = static_cast<char *>(out->data) + (size_t)co * out->component_bytes;

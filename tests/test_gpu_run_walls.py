@@ -3,8 +3,8 @@ import numpy as np
 import pytest
 
 import cubismnova_amd as cnv
-from tests.helpers import assert_same
-from tests.test_gpu_cols import build
+from tests.helpers import assert_same, cells_of, face_bc_lists
+from tests.test_gpu_cols import KIND, MIXED, PARTLY, build
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +30,59 @@ def test_symmetry_factor_below_single_precision(gpu, axis):
     """A Symmetry factor that is not zero in the list and zero in the grid's type
     mirrors to a ghost of zero, in both steps of a launch."""
     run_and_singles((4, 4, 4), (32, 32, 32), np.float32, [[(3, axis, 0, 1e-60), (3, axis, 1, -1e-60)]], 4)
+
+
+def relist(g, lists):
+    """The grid's lists replaced, a list of faces per component."""
+    for c, faces in enumerate(lists):
+        for b, lst in face_bc_lists(g.nblocks, faces).items():
+            bi = (b % g.nblocks[0], (b // g.nblocks[0]) % g.nblocks[1], b // (g.nblocks[0] * g.nblocks[1]))
+            g.setBC(bi, [KIND[k](d, s, v) if k in (2, 3) else KIND[k](d, s) for k, d, s, v in lst], comp=c)
+
+
+CHANGED = [[(k, d, s, v - 0.375) if k == 2 else (k, d, s, v) for k, d, s, v in MIXED],  # other constants
+           [(1, 0, 0, 0.0), (2, 0, 1, 0.25), (3, 1, 0, 0.5), (1, 1, 1, 0.0), (3, 2, 0, -1.0), (2, 2, 1, 2.0)]]  # other rules
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("nb,n", [((2, 2, 2), (20, 20, 20)), ((5, 5, 5), (24, 24, 24)), ((6, 5, 4), (32, 32, 32))],
+                         ids=["lds tiles", "domain tiles", "block tiles"])
+def test_recorded_run_follows_the_lists(gpu, dtype, nb, n):
+    """Lists changed after a run was recorded (as long as before, one rule per
+    domain face): a replay takes them from the prepared grids, in its launches of
+    several steps as in its single ones.  A face of two rules turns it into NaN."""
+    first, steps = [MIXED, [], PARTLY], 7
+    u, t, v, w = (build(nb, n, dtype, 107, first)[0] for _ in range(4))
+    start = [u.download(c) for c in range(3)]
+    dt = 0.1 / max(nb[d] * n[d] for d in range(3)) ** 2
+    norms, want = cnv.DeviceBuffer(8 * steps), cnv.DeviceBuffer(8 * steps)
+    s = cnv.Stream()
+    cnv.diffusion_run(u, t, steps, dt, norms, stream=s)
+    s.synchronize()
+    g = cnv.Graph(s).capture()
+    cnv.diffusion_run(u, t, steps, dt, norms, stream=s)
+    g.end()
+
+    def replay():
+        for x in (u, v):
+            for c in range(3):
+                x.upload(c, start[c])
+        g.launch()
+        s.synchronize()
+
+    for lists in [first] + [[x, [], PARTLY] for x in CHANGED]:
+        for x in (u, t, v, w):
+            relist(x, lists)
+            x.prepare()
+        replay()
+        assert cnv.diffusion_run(v, w, steps, dt, want) is w
+        for c in range(3):
+            assert_same(cells_of(t.download(c), nb, n, t.block_stride), cells_of(w.download(c), nb, n, w.block_stride),
+                        "component %d" % c)
+        assert np.array_equal(norms.download(np.float64, steps), want.download(np.float64, steps))
+    for x in (u, t):
+        lst = x.getBC((0, 0, 0))
+        x.setBC((0, 0, 0), [cnv.Dirichlet(0, 0, 9.0)] + lst[1:])
+        x.prepare()
+    replay()
+    assert np.any(np.isnan(t.download(0)))

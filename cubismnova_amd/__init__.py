@@ -7,6 +7,7 @@ every compute call goes through the C ABI of libcubismnova_amd.so
 block layout; numpy arrays are only the host side of uploads and downloads.
 """
 import ctypes
+import threading
 
 import numpy as np
 
@@ -300,7 +301,7 @@ class Cartesian:
         self.nblocks_total = nb[0] * nb[1] * nb[2]
         self._mesh = _Mesh(b, e, [nb[k] * bc[k] for k in range(3)])
         self._bcs = {}
-        self._red = None
+        self._red = threading.local()
 
     @classmethod
     def from_tensor(cls, t, nblocks, block_cells, begin=0.0, end=1.0, ncomp=1, entity="cell"):
@@ -445,11 +446,12 @@ class Cartesian:
         return out, list(ext)
 
     def _reductions(self):
-        """Device memory of this grid's reduction results, kept with the
-        partial sums the grid holds (allocated by the first reduction)."""
-        if self._red is None:
-            self._red = DeviceBuffer(24)
-        return self._red
+        """Device memory of this grid's reduction results: a buffer per thread
+        (a call reads its results after it queued them, when another thread's
+        may be queued behind), allocated by the thread's first reduction."""
+        if not hasattr(self._red, "buf"):
+            self._red.buf = DeviceBuffer(24)
+        return self._red.buf
 
     def __del__(self):
         try:

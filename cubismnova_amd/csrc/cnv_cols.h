@@ -48,6 +48,7 @@ struct ColShape {
     int nzc, zchunk; // z chunks per block, planes per chunk
     int nbt;         // blocks
     int ntiles;      // components * blocks * z chunks
+    WgGrid wgs;
     FastDiv dlanes, dvx, dnzc, dnbt, dnbx, dnby;
 };
 
@@ -73,19 +74,23 @@ inline int col_zchunk(const Geom &G, int ncomp, int vec)
     return (int)(z < 1 ? 1 : z > G.n[2] ? G.n[2] : z);
 }
 
-// zchunk planes per lane; false when the launch does not fit 32-bit tiles
-inline bool col_shape(const Geom &G, int ncomp, int vec, int zchunk, ColShape &s, long long &nwg)
+// zchunk planes per lane; false when the launch does not fit 32-bit tiles or
+// lanes of a plane
+inline bool col_shape(const Geom &G, int ncomp, int vec, int zchunk, ColShape &s)
 {
     s.vx = G.n[0] / vec;
+    if ((long long)s.vx * G.n[1] >= (1LL << 31) - kColWG)
+        return false;
     s.lanes = s.vx * G.n[1];
     const long long nbt = (long long)G.nb[0] * G.nb[1] * G.nb[2];
     s.nzc = (G.n[2] + zchunk - 1) / zchunk;
     s.zchunk = (G.n[2] + s.nzc - 1) / s.nzc; // even chunks
     s.nzc = (G.n[2] + s.zchunk - 1) / s.zchunk;
     const long long ntiles = nbt * ncomp * s.nzc;
-    nwg = (ntiles * s.lanes + kColWG - 1) / kColWG;
-    if (ntiles >= (1LL << 31) || nwg >= (1LL << 31))
+    const long long nwg = (ntiles * s.lanes + kColWG - 1) / kColWG;
+    if (ntiles >= (1LL << 31) - kColWG || nwg >= (1LL << 31) - kColWG)
         return false;
+    s.wgs = wg_grid(nwg);
     s.nbt = (int)nbt;
     s.ntiles = (int)ntiles;
     s.dlanes = fast_div((unsigned)s.lanes);
@@ -108,7 +113,7 @@ __device__ inline ColLane col_lane(const ColShape &s, const Geom &G)
 {
     ColLane c;
     // the workgroup's first lane by scalar arithmetic, then 32 bits per lane
-    const long long base = (long long)xcd_remap(blockIdx.x, gridDim.x) * kColWG;
+    const long long base = (long long)xcd_remap(wg_index(s.wgs), s.wgs.count) * kColWG;
     const int t0 = base < (1LL << 31) ? fdiv((int)base, s.dlanes) : (int)(base / s.lanes);
     const int r = (int)(base - (long long)t0 * s.lanes) + (int)threadIdx.x;
     const int dt = fdiv(r, s.dlanes);

@@ -266,6 +266,23 @@ __device__ inline int xcd_remap(int i, int n)
     return x * q + (x < r ? x : r) + local;
 }
 
+// Workgroups of a launch that may hold 2^32 threads and more (one dimension of a
+// launch holds fewer, and more are cut off without an error): rows of at most
+// 2^23 workgroups of up to 256 threads, a few workgroups more than n in the last.
+struct WgGrid {
+    int x, count; // workgroups of a row and of all rows
+
+    dim3 dim() const { return dim3((unsigned)x, (unsigned)(count / x)); }
+};
+
+inline WgGrid wg_grid(long long n)
+{
+    const long long rows = (n + (1 << 23) - 1) >> 23, x = (n + rows - 1) / rows;
+    return {(int)x, (int)(x * rows)};
+}
+
+__device__ inline int wg_index(const WgGrid &g) { return (int)blockIdx.y * g.x + (int)blockIdx.x; }
+
 // Source of the ghost layers of one block face.  Ghost layer l (1 = next to
 // the face) at in-face offset i reads p[(li0 + lstep*l) * dstride + i], then
 // copies it (mode 0), scales it by s (mode 1, Symmetry), or is the constant s

@@ -190,7 +190,8 @@ __device__ inline void lab_region(const LabArgs<T> &a, const int B[3], const int
 // for the x ghosts (three cells of a 128-byte line) and, small, by the rules.
 constexpr int kLabPer = 4;
 
-template <typename T>
+// ROWS: a row of workgroups per block, where one dimension does not hold them all.
+template <typename T, bool ROWS>
 __global__ __launch_bounds__(256) void k_lab(const LabArgs<T> a)
 {
     __shared__ LabRegion<T> reg[27];
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(256) void k_lab(const LabArgs<T> a)
     int B[3], n = 0;
     // the workgroups of a block, and of neighbouring blocks, on one XCD
     const int wg = xcd_remap(blockIdx.x, gridDim.x);
-    const int slot = wg / a.wgslot, wl = wg - slot * a.wgslot;
+    const int slot = ROWS ? blockIdx.y : wg / a.wgslot, wl = ROWS ? blockIdx.x : wg - slot * a.wgslot;
     if (a.single) {
         B[0] = a.block[0];
         B[1] = a.block[1];
@@ -366,10 +367,14 @@ static int launch_lab_t(const cnv_grid_s *g, int comp, const cnv_stencil &s, boo
     a.zchunk = (passes + nzc - 1) / nzc * per;
     nzc = (a.L[2] + a.zchunk - 1) / a.zchunk;
     const long long gx = wgxy * nzc;
-    if (gx * nslots > 0x7fffffffLL)
+    const long long most = (1LL << 24) - 1; // a dimension of 2^32 threads or more is cut off without an error
+    if (gx > most)
         return fail(CNV_ERR_UNSUPPORTED, "lab too large");
     a.wgslot = (int)gx;
-    hipLaunchKernelGGL(k_lab<T>, dim3((unsigned)(gx * nslots)), dim3(256), 0, st, a);
+    if (gx * nslots <= most)
+        hipLaunchKernelGGL((k_lab<T, false>), dim3((unsigned)(gx * nslots)), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_lab<T, true>), dim3((unsigned)gx, (unsigned)nslots), dim3(256), 0, st, a);
     CNV_HIP(hipGetLastError());
     return CNV_OK;
 }

@@ -340,7 +340,7 @@ static bool run2_layout(const cnv_grid_s *u, Run2Args &a, int ncomp, int zchunk)
         nt *= a.nt[d];
     }
     a.zchunk = zchunk;
-    if (nt >= (1LL << 30))
+    if (nt >= (1LL << 32) / kRun2WG - 4) // (and the deferred sums: fewer than 2^32 threads)
         return false;
     a.ntiles = (int)nt;
     return true;

@@ -146,7 +146,7 @@ __global__ __launch_bounds__(kColWG) void k_stencil7_cols(const S7Args a, const 
     using V = VecT<T, VEC>;
     __shared__ double red[kColWG / 64];
     const int tid = threadIdx.x;
-    if (blockIdx.x == 0)
+    if (wg_index(s.wgs) == 0)
         for (int k = 0; k < 2; ++k)
             if (a.prev_p[k])
                 wg_sum_partials<kColWG>(a.prev_p[k], a.prev_n[k], a.prev_out[k], red);
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kColWG) void k_stencil7_cols(const S7Args a, const 
             red[tid >> 6] = acc;
         __syncthreads();
         if (tid == 0)
-            a.partials[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+            a.partials[wg_index(s.wgs)] = ((red[0] + red[1]) + red[2]) + red[3];
     }
 }
 
@@ -330,12 +330,12 @@ static bool dispatch_spec(const S7Args &a, int edge, int wg, int ntiles, hipStre
 }
 
 template <typename T, int VEC, int MODE, bool SUMSQ>
-static void launch_cols(const S7Args &a, const ColShape &s, unsigned nwg, bool bc, hipStream_t st)
+static void launch_cols(const S7Args &a, const ColShape &s, bool bc, hipStream_t st)
 {
     if (bc)
-        hipLaunchKernelGGL((k_stencil7_cols<T, VEC, MODE, SUMSQ, true>), dim3(nwg), dim3(kColWG), 0, st, a, s);
+        hipLaunchKernelGGL((k_stencil7_cols<T, VEC, MODE, SUMSQ, true>), s.wgs.dim(), dim3(kColWG), 0, st, a, s);
     else
-        hipLaunchKernelGGL((k_stencil7_cols<T, VEC, MODE, SUMSQ, false>), dim3(nwg), dim3(kColWG), 0, st, a, s);
+        hipLaunchKernelGGL((k_stencil7_cols<T, VEC, MODE, SUMSQ, false>), s.wgs.dim(), dim3(kColWG), 0, st, a, s);
 }
 
 // The sizes the column kernel takes: gx groups of 256 cells per block, gy blocks
@@ -362,23 +362,22 @@ static int run_cols(S7Args &a, int ncomp, hipStream_t st, bool finalize, int *np
         return fail(CNV_ERR_SIZE, "grid needs more norm partials than the scratch array holds");
     const int vec = col_vec(n[0], sizeof(T));
     ColShape s;
-    long long nwg = 0;
-    if (!col_shape(a.G, ncomp, vec, col_zchunk(a.G, ncomp, vec), s, nwg))
+    if (!col_shape(a.G, ncomp, vec, col_zchunk(a.G, ncomp, vec), s))
         return fail(CNV_ERR_UNSUPPORTED, "grid too large for the generic stencil kernel");
     bool bc = false;
     for (int c = 0; c < ncomp; ++c)
         bc = bc || a.has_bc[c];
     if (vec == 1)
-        launch_cols<T, 1, MODE, SUMSQ>(a, s, (unsigned)nwg, bc, st);
+        launch_cols<T, 1, MODE, SUMSQ>(a, s, bc, st);
     else if (vec == 2)
-        launch_cols<T, 2, MODE, SUMSQ>(a, s, (unsigned)nwg, bc, st);
+        launch_cols<T, 2, MODE, SUMSQ>(a, s, bc, st);
     else if constexpr (sizeof(T) == 4)
-        launch_cols<T, 4, MODE, SUMSQ>(a, s, (unsigned)nwg, bc, st);
+        launch_cols<T, 4, MODE, SUMSQ>(a, s, bc, st);
     CNV_HIP(hipGetLastError());
     if (nparts)
-        *nparts = (int)nwg;
+        *nparts = s.wgs.count;
     if (SUMSQ && finalize) {
-        hipLaunchKernelGGL(k_finalize_sum, dim3(1), dim3(1024), 0, st, a.partials, (int)nwg, a.sumsq);
+        hipLaunchKernelGGL(k_finalize_sum, dim3(1), dim3(1024), 0, st, a.partials, s.wgs.count, a.sumsq);
         CNV_HIP(hipGetLastError());
     }
     return CNV_OK;

@@ -323,7 +323,7 @@ static bool tile_layout(const cnv_grid_s *u, TileArgs &a, int cx, int cy, int cz
         a.dn[d] = fast_div((unsigned)G.n[d]);
         nt *= a.nt[d];
     }
-    if (nt >= (1LL << 30))
+    if (nt >= (1LL << 32) / 1024 - 4) // (and the deferred sums: fewer than 2^32 threads)
         return false;
     a.ntiles = (int)nt;
     return true;

@@ -270,8 +270,7 @@ static int w5_cols(const W5Args &a, hipStream_t st)
     const long long vectors = gy * ((long long)n[0] / vec * n[1] * n[2]);
     const int z = (int)std::min<long long>(16, std::max<long long>(1, vectors / (sizeof(T) == 4 ? 409600 : 163840)));
     ColShape s;
-    long long nwg = 0;
-    if (!col_shape(a.G, a.ncomp, vec, std::min(z, n[2]), s, nwg))
+    if (!col_shape(a.G, a.ncomp, vec, std::min(z, n[2]), s))
         return fail(CNV_ERR_UNSUPPORTED, "grid too large for the generic WENO5 kernel");
     bool bc = false;
     for (int c = 0; c < a.ncomp; ++c)
@@ -279,9 +278,9 @@ static int w5_cols(const W5Args &a, hipStream_t st)
     auto go = [&](auto v) {
         constexpr int VEC = decltype(v)::value;
         if (bc)
-            hipLaunchKernelGGL((k_weno5_cols<T, VEC, true>), dim3((unsigned)nwg), dim3(kColWG), 0, st, a, s);
+            hipLaunchKernelGGL((k_weno5_cols<T, VEC, true>), s.wgs.dim(), dim3(kColWG), 0, st, a, s);
         else
-            hipLaunchKernelGGL((k_weno5_cols<T, VEC, false>), dim3((unsigned)nwg), dim3(kColWG), 0, st, a, s);
+            hipLaunchKernelGGL((k_weno5_cols<T, VEC, false>), s.wgs.dim(), dim3(kColWG), 0, st, a, s);
     };
     if (vec == 1)
         go(std::integral_constant<int, 1>());

@@ -552,21 +552,24 @@ X2Tune x2_tune(int dtype, int edge, bool *pinned = nullptr)
 }
 
 // Tiles a launch needs to fill the GPU with the built-in workgroup size
-// (fewer where a tile has more waves or more LDS).
+// (fewer where a tile has more waves or more LDS); FP32 on 16^3 blocks comes here
+// with a pinned tile only.
 int x2_enough(int dtype, int edge)
 {
     if (edge == 32)
         return dtype == CNV_F64 ? 400 : 600;
-    return dtype == CNV_F64 ? 800 : 1500;
+    return 800;
 }
 
 // z-chunks that can be pinned: 8, 16 and 32 planes (up to the block edge);
-// chunks of 2 and 4 planes are compiled for small grids
+// chunks of 2 and 4 planes are compiled for small grids, which take the built-in
+// workgroup size
 inline bool x2_zchunk_ok(int zc) { return zc == 8 || zc == 16 || zc == 32; }
 
 template <typename T, int N, int WG, bool WALL>
 bool x2_launch1(const X2Args &a, int zc, int ntiles, hipStream_t st)
 {
+    constexpr bool SHALLOW = N == 32 ? WG == 256 : sizeof(T) == 8 && WG == 128;
     if constexpr (X2Shape<T, N, WG>::valid) {
         auto go = [&](auto z) {
             hipLaunchKernelGGL((k_stencil7x2<T, N, WG, decltype(z)::value, WALL>), dim3(ntiles), dim3(WG), 0, st, a);
@@ -574,9 +577,13 @@ bool x2_launch1(const X2Args &a, int zc, int ntiles, hipStream_t st)
         };
         switch (zc) {
         case 2:
-            return go(std::integral_constant<int, 2>());
+            if constexpr (SHALLOW)
+                return go(std::integral_constant<int, 2>());
+            break;
         case 4:
-            return go(std::integral_constant<int, 4>());
+            if constexpr (SHALLOW)
+                return go(std::integral_constant<int, 4>());
+            break;
         case 8:
             return go(std::integral_constant<int, 8>());
         case 16:

@@ -25,6 +25,38 @@ def run_and_singles(nb, n, dtype, lists, steps, seed=101):
     assert np.max(np.abs(gn - wn) / wn) <= 1e-13
 
 
+THREE = [MIXED, [], PARTLY]
+
+
+@pytest.mark.parametrize("nb,edge,dtype,lists", [
+    ((4, 4, 4), 32, np.float32, [[]]),           # two planes per tile
+    ((4, 4, 4), 32, np.float32, [MIXED]),
+    ((2, 3, 2), 32, np.float64, [MIXED]),        # two planes
+    ((6, 5, 4), 32, np.float32, THREE),          # a component without lists among walled ones
+    ((6, 5, 4), 32, np.float64, THREE),
+    ((5, 5, 5), 16, np.float64, THREE),
+    ((5, 5, 5), 16, np.float64, [[], [], []]),
+    ((1, 6, 8), 32, np.float32, [MIXED]),        # one block between two walls
+    ((8, 1, 6), 32, np.float64, [MIXED]),
+    ((8, 6, 1), 32, np.float32, [MIXED, PARTLY]),
+])
+def test_block_tiles(gpu, nb, edge, dtype, lists):
+    """Grids larger than the LDS tiles take: the kernel on block tiles, at its
+    shallowest, with several components and with walls a block apart."""
+    run_and_singles(nb, (edge,) * 3, dtype, lists, 7)
+
+
+@pytest.mark.parametrize("edge,dtype", [(16, np.float32), (16, np.float64), (32, np.float32)])
+@pytest.mark.parametrize("lists", [[[], [], []], THREE], ids=["periodic", "walls"])
+def test_block_tiles_pinned_on_a_small_grid(gpu, edge, dtype, lists):
+    saved = cnv.tune_diffusion_run(dtype, edge)
+    cnv.set_tune_diffusion_run(dtype, edge, saved[0], 8)
+    try:
+        run_and_singles((2, 3, 2), (edge,) * 3, dtype, lists, 7)
+    finally:
+        cnv.set_tune_diffusion_run(dtype, edge, *saved)
+
+
 @pytest.mark.parametrize("axis", [0, 1, 2])
 def test_symmetry_factor_below_single_precision(gpu, axis):
     """A Symmetry factor that is not zero in the list and zero in the grid's type

@@ -345,7 +345,8 @@ struct cnv_batch_s {
     // width), workgroup size
     bool one = true;
     int one_wg = 256;
-    bool one_deep = false; // many WENO5 blocks: deeper items (one_zdepth)
+    bool one_deep = false;   // many WENO5 blocks: deeper items (one_zdepth)
+    bool one_tail16 = false; // a few 16^3 blocks of diffusion are the longest items
     std::map<std::pair<int, int>, int> zmap;
     std::vector<BItem> one_items;
     std::vector<BUnit> units;
@@ -627,23 +628,27 @@ static int launch_generic(cnv_batch_s *b, hipStream_t st)
 // Planes per item of the single launch for a grid: the tuned depth of its
 // (block edge, ghost width), else by its operator.  A WENO5 item marches its
 // planes at about 2 us each, so a 32-plane item is 75 us of one workgroup: the
-// launch's tail, and all of a small batch.  WENO5 and 16^3 blocks take 8 planes
-// (16 when the batch holds 1024 32^3 blocks of WENO5: the planes that chunks read
-// twice then cost more than the tail), diffusion on 32^3 blocks whole blocks.
-// Us per step with 32 / 16 / 8 WENO5 planes: 96 grids (2333 32^3 blocks of WENO5)
-// 716 / 683 / 693, 35 grids (354 blocks) 187 / 150 / 129, 35 small grids 78 / 43 /
-// 31; diffusion on 32^3 with 8 planes instead of 32: 129 -> 140 and no gain
-// elsewhere; 12 grids of 16^3 diffusion with 16 / 8 planes 14.9 / 9.7, the 96 grids
-// 641 / 673 (both operators on 16^3).  Other shapes take up to 32 or 8 planes by
-// their edge, halved until the tile fits: 12 grids of WENO5 on 32x32x20 blocks 65
-// with the 5 planes of that, 118 with 8, whose 62 KB leave two workgroups per CU.
+// launch's tail, and all of a small batch.  WENO5 takes 8 planes (16 when the
+// batch holds 1024 32^3 blocks of it: the four extra planes a chunk reads then
+// cost more than the tail), diffusion whole blocks.  Us per step with 32 / 16 / 8
+// WENO5 planes: 96 grids (2333 32^3 blocks of WENO5) 716 / 683 / 693, 35 grids (354
+// blocks) 187 / 150 / 129, 35 small grids 78 / 43 / 31; diffusion items of 8 planes
+// instead of 32: 129 -> 140 and no gain elsewhere.
+//   Diffusion on 16^3 blocks is the tail where the batch holds nothing longer, and
+// takes 8 planes there while all of its units run at once.  Us with 16 / 8 planes:
+// 64 such blocks 13.3 / 8.6, 1536 19.4 / 16.0, 2048 20.2 / 17.4, 3072 23.6 / 29.9;
+// beside two 32^3 blocks or eight 16^3 blocks of WENO5 level (21.8 / 21.7, 22.9 /
+// 23.1), from 1024 blocks on slower (25.3 / 26.6, 24.6 / 25.6).
+//   Other shapes take up to 32 or 8 planes by their edge, halved until the tile
+// fits: 12 grids of WENO5 on 32x32x20 blocks 65 us with the 5 planes of that, 118
+// with 8, whose 62 KB leave two workgroups per CU.
 static int one_zdepth(const cnv_batch_s *b, const cnv_batch_item &it)
 {
     const cnv_grid_s *g = it.in;
     const std::pair<int, int> key(class_key_edge(g), it.ghost);
     int nz = key.first >= 32 ? 32 : 8;
-    if (marchable(it) && (it.op == CNV_OP_WENO5 || key.first == 16))
-        nz = b->one_deep ? 16 : 8;
+    if (marchable(it))
+        nz = it.op == CNV_OP_WENO5 ? (b->one_deep ? 16 : 8) : key.first == 16 ? (b->one_tail16 ? 8 : 16) : 32;
     if (b->zmap.count(key))
         nz = b->zmap.at(key);
     return std::max(1, std::min(nz, g->desc.block_cells[2]));
@@ -680,12 +685,19 @@ static int build_one(cnv_batch_s *b)
         BItem item;
     };
     std::vector<Tmp> all;
-    long long weno_cells = 0;
-    for (const auto &it : b->src)
+    long long weno_cells = 0, blocks16 = 0;
+    bool longer = false; // than 16^3 cells of diffusion
+    for (const auto &it : b->src) {
+        const int *n = it.in->desc.block_cells;
+        const long long cells = (long long)n[0] * n[1] * n[2], blocks = it.in->nblocks_total * it.in->desc.ncomp;
         if (marchable(it) && it.op == CNV_OP_WENO5)
-            weno_cells += it.in->nblocks_total * it.in->desc.ncomp * it.in->desc.block_cells[0] *
-                          it.in->desc.block_cells[1] * it.in->desc.block_cells[2];
+            weno_cells += blocks * cells;
+        longer = longer || it.op == CNV_OP_WENO5 || cells > 16 * 16 * 16;
+        if (marchable(it) && n[0] == 16)
+            blocks16 += blocks;
+    }
     b->one_deep = weno_cells >= 1024LL * 32 * 32 * 32;
+    b->one_tail16 = !longer && blocks16 <= 2000;
     for (size_t gi = 0; gi < b->src.size(); ++gi) {
         const cnv_batch_item &it = b->src[gi];
         const cnv_grid_s *g = it.in;

@@ -33,3 +33,15 @@ def test_units_of_a_small_batch(gpu, nb, n, op, units):
             assert np.max(np.abs(got - want)) <= 1e-6 * np.max(np.abs(want))
         else:
             assert np.array_equal(got, want)
+
+
+def test_16_cubed_diffusion_beside_longer_items(gpu):
+    """Whole blocks where another item takes longer than they do."""
+    made = [build(nb, n, np.float32, 37, [MIXED])[0] for nb, n in (((2, 2, 1), (16,) * 3), ((1, 2, 1), (32,) * 3))]
+    outs, refs = ([cnv.Cartesian(g.nblocks, g.block_cells, dtype=np.float32) for g in made] for _ in range(2))
+    b = cnv.Batch([(g, o, "diffusion", 1, 1e-6) for g, o in zip(made, outs)])
+    assert b.form() == (cnv.Batch.SINGLE, 1 + 2)
+    b.run()
+    for g, o, r in zip(made, outs, refs):
+        cnv.diffusion_step(g, r, 1e-6)
+        assert np.array_equal(o.download(0), r.download(0))

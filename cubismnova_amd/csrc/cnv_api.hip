@@ -64,13 +64,13 @@ int ensure_rules(cnv_grid_s *g, const hipStream_t *run)
         if (first || f.longest > 0)
             g->rules_host[c] = face_rules(f);
     }
-    if (!first) // kernels still queued on any stream may read them
-        CNV_HIP(hipDeviceSynchronize());
     if (run && g->nslabs <= kX2MaxComp) { // (a copy is 20 us of the first run on a grid, this 4)
         const int rc = launch_rules(g, *run);
         if (rc != CNV_OK)
             return rc;
     } else {
+        if (!first) // kernels still queued on any stream may read them
+            CNV_HIP(hipDeviceSynchronize());
         CNV_HIP(hipMemcpy(g->rules, g->rules_host.data(), sizeof(FaceRules) * (size_t)g->nslabs,
                           hipMemcpyHostToDevice));
     }
@@ -131,7 +131,7 @@ int ensure_bc_table(cnv_grid_s *g, int comp)
     CNV_HIP(hipMemcpy(t.heads, image.get(), hb + eb, hipMemcpyHostToDevice));
     t.any = ne > 0;
     t.version = g->bc_version;
-    return g->rules_version == ~0ull ? CNV_OK : ensure_rules(g, nullptr); // both or none follow the lists
+    return g->rules_recorded ? ensure_rules(g, nullptr) : CNV_OK; // recorded runs read both
 }
 
 // Every block's BC list resolved for a stencil that reads both sides (-1, 2)

@@ -124,6 +124,7 @@ struct cnv_grid_s {
     cnv::FaceRules *rules = nullptr;
     std::vector<cnv::FaceRules> rules_host;
     uint64_t rules_version = ~0ull;
+    bool rules_recorded = false; // some recorded launch reads them
 
     // z metric of a stretched mesh (per global z cell), set on first use
     double *czm_dev = nullptr;

@@ -699,23 +699,26 @@ int launch_rules(cnv_grid_s *g, hipStream_t st)
 
 // The rules of g's first ncomp components for launches on st that read g.  The
 // device's copies follow the lists in every run, so that a run can be recorded
-// after it was called once, and with them a table that single steps had built.
+// after it was called once; once one was, the table that its single steps read
+// follows with them.
 int run_rules(cnv_grid_s *g, int ncomp, hipStream_t st, RunRules &r)
 {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (st)
         (void)hipStreamIsCapturing(st, &cs);
     std::lock_guard<std::mutex> lk(g->mtx);
-    if (cs != hipStreamCaptureStatusNone && g->rules_version != g->bc_version)
+    const bool rec = cs != hipStreamCaptureStatusNone;
+    if (rec && g->rules_version != g->bc_version)
         return fail(CNV_ERR_INVALID, "BC lists changed since this grid's last run: run once before recording");
     int rc = ensure_rules(g, &st);
     for (int c = 0; c < ncomp && rc == CNV_OK; ++c) {
         const FaceInfo &f = face_info(g, c);
         r.val[c] = face_rules(f);
-        r.p[c] = cs != hipStreamCaptureStatusNone && f.longest > 0 ? g->rules + c : nullptr;
-        if (g->tables[c].heads)
+        r.p[c] = rec && f.longest > 0 ? g->rules + c : nullptr;
+        if (g->rules_recorded && g->tables[c].heads)
             rc = ensure_bc_table(g, c);
     }
+    g->rules_recorded = g->rules_recorded || rec;
     return rc;
 }
 

@@ -81,8 +81,8 @@ CHANGED = [[(k, d, s, v - 0.375) if k == 2 else (k, d, s, v) for k, d, s, v in M
                          ids=["lds tiles", "domain tiles", "block tiles"])
 def test_recorded_run_follows_the_lists(gpu, dtype, nb, n):
     """Lists changed after a run was recorded (as long as before, one rule per
-    domain face): a replay takes them from the prepared grids, in its launches of
-    several steps as in its single ones.  A face of two rules turns it into NaN."""
+    domain face): a replay takes them from the grids, prepared or run meanwhile, in
+    its launches of several steps as in its single ones.  A face of two rules turns it into NaN."""
     first, steps = [MIXED, [], PARTLY], 7
     u, t, v, w = (build(nb, n, dtype, 107, first)[0] for _ in range(4))
     start = [u.download(c) for c in range(3)]
@@ -102,10 +102,14 @@ def test_recorded_run_follows_the_lists(gpu, dtype, nb, n):
         g.launch()
         s.synchronize()
 
-    for lists in [first] + [[x, [], PARTLY] for x in CHANGED]:
+    for k, lists in enumerate([first] + [[x, [], PARTLY] for x in CHANGED + [MIXED]]):
         for x in (u, t, v, w):
             relist(x, lists)
-            x.prepare()
+            if k % 2 == 0:
+                x.prepare()
+        if k % 2 == 1:  # a run of these grids does it too, here one of fused launches alone
+            cnv.diffusion_run(u, t, 4, dt, stream=s)
+            s.synchronize()
         replay()
         assert cnv.diffusion_run(v, w, steps, dt, want) is w
         for c in range(3):

@@ -238,8 +238,11 @@ int cnv_diffusion_step_noalloc(const cnv_grid_desc *desc, const void *u, void *u
  * grids that are periodic (no BC list) or whose BC lists give each domain face
  * one rule on all its blocks (periodic on both sides of an axis, or per side
  * Dirichlet, Symmetry of nonzero sign or Absorbing), runs of four steps and more
- * go four or two steps per launch on small and medium grids of any block shape
- * and two on every grid of 16^3 or 32^3 blocks.  The loop of the reference's time stepping over Field.h:457-512 / FieldOperator.h. */
+ * go four or two steps per launch on small grids and two on larger ones, whatever
+ * the block shape.  A run is refused before its first launch where a single step
+ * would be (except that periodic grids of 16^3 or 32^3 blocks take more than 8
+ * components for a multiple of four steps).  The loop of the reference's time
+ * stepping over Field.h:457-512 / FieldOperator.h. */
 int cnv_diffusion_run(cnv_grid u, cnv_grid tmp, int nsteps, double nu_dt, double *norms, cnv_stream s);
 
 /* Fifth-order WENO face states (Jiang & Shu, J. Comput. Phys. 126:202-228,
@@ -333,8 +336,9 @@ typedef struct {
  * A e = r with u's BCs made homogeneous, adds e to u in FP64 and recomputes
  * the FP64 defect.  refine = 0: plain sweeps in u's dtype, work of u's dtype
  * with 2 components.  The launches go to stream s, which the host waits for
- * once per cycle; the relative residual after cycle c goes to history[c]
- * (history[0] = initial).  Calls on the same grids must not overlap. */
+ * once per cycle (solves of several threads on the NULL stream share it); the
+ * relative residual after cycle c goes to history[c] (history[0] = initial).
+ * Calls on the same grids must not overlap. */
 int cnv_jacobi_solve(cnv_grid u, cnv_grid f, cnv_grid work, const cnv_solve_opts *opts, cnv_solve_info *info,
                      double *history, int history_cap, cnv_stream s);
 

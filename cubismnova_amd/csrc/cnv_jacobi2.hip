@@ -380,21 +380,25 @@ __global__ __launch_bounds__(WG) void k_jacobi2(const J2Args a)
     const bool ring_skip =
         MIR && (SCALAR ? mirrored(shx[0], shy[0]) : (role == 1 ? mirrored(hx + ringv, hy) : mirrored(hx, hy)));
     // the ghost u' this thread writes for a mirror or edge face next to
-    // the tile: the factor (0: none) for the cell left of its first cell
-    // (x0 = 0), right of its last (x0 = NX - VEC), and for the row below
-    // row 0 / above row TY - 1 of its cells
-    auto ghost_factor = [&](int d, int side, bool at_edge) -> T {
-        if (!MIR || !at_edge || a.fm[d][side] < FM_MIRROR)
-            return (T)0;
-        return a.fm[d][side] == FM_MIRROR ? (T)a.fv[d][side] : (T)1;
+    // the tile, times the factor (which may be 0 in T): for the cell left of its
+    // first cell (x0 = 0), right of its last (x0 = NX - VEC), and for the row
+    // below row 0 / above row TY - 1 of its cells
+    struct Ghost {
+        bool on;
+        T f;
     };
-    const T gxl = ghost_factor(0, 0, bx == 0 && x0 == 0);
-    const T gxr = ghost_factor(0, 1, bx == nbx - 1 && x0 + VEC == NX);
-    const T gyl = ghost_factor(1, 0, by == 0 && y0 == 0);
-    const T gyh = ghost_factor(1, 1, by == nby - 1 && y0 + TY == NX);
+    auto ghost_factor = [&](int d, int side, bool at_edge) -> Ghost {
+        if (!MIR || !at_edge || a.fm[d][side] < FM_MIRROR)
+            return {false, (T)0};
+        return {true, a.fm[d][side] == FM_MIRROR ? (T)a.fv[d][side] : (T)1};
+    };
+    const Ghost gxl = ghost_factor(0, 0, bx == 0 && x0 == 0);
+    const Ghost gxr = ghost_factor(0, 1, bx == nbx - 1 && x0 + VEC == NX);
+    const Ghost gyl = ghost_factor(1, 0, by == 0 && y0 == 0);
+    const Ghost gyh = ghost_factor(1, 1, by == nby - 1 && y0 + TY == NX);
     // sweep two at the first / last plane of a z mirror or edge face reads
     // its ghost u' as this factor times u' of that plane
-    const T gzl = ghost_factor(2, 0, true), gzh = ghost_factor(2, 1, true);
+    const Ghost gzl = ghost_factor(2, 0, true), gzh = ghost_factor(2, 1, true);
     // f at the held ring cells (planes of the tile only: z inside the grid)
     auto fetch_fring = [&](const ZPart &z, V &Fr) {
         if constexpr (SCALAR) {
@@ -524,12 +528,12 @@ __global__ __launch_bounds__(WG) void k_jacobi2(const J2Args a)
                 *reinterpret_cast<V *>(B + (y + 1) * PA + VEC + x0) = res;
                 // ghost u' past a mirror or edge face, for the tile's planes
                 if (MIR && j >= 1 && j <= nzt) {
-                    if (gxl != (T)0)
-                        B[(y + 1) * PA + VEC - 1] = res.v[0] * gxl;
-                    if (gxr != (T)0)
-                        B[(y + 1) * PA + VEC + NX] = res.v[VEC - 1] * gxr;
-                    if ((y == 0 && gyl != (T)0) || (y == TY - 1 && gyh != (T)0)) {
-                        const T gf = y == 0 ? gyl : gyh;
+                    if (gxl.on)
+                        B[(y + 1) * PA + VEC - 1] = res.v[0] * gxl.f;
+                    if (gxr.on)
+                        B[(y + 1) * PA + VEC + NX] = res.v[VEC - 1] * gxr.f;
+                    if ((y == 0 && gyl.on) || (y == TY - 1 && gyh.on)) {
+                        const T gf = y == 0 ? gyl.f : gyh.f;
                         V gv;
 #pragma unroll
                         for (int v = 0; v < VEC; ++v)
@@ -580,7 +584,7 @@ __global__ __launch_bounds__(WG) void k_jacobi2(const J2Args a)
             const int q = p - 1;
             T *oq = obase + blk * bstride + SXY * q;
             const int gq = bz * NZ + q;
-            const T fzl = gq == 0 ? gzl : (T)0, fzh = gq == NGZ - 1 ? gzh : (T)0;
+            const bool ozl = gzl.on && gq == 0, ozh = gzh.on && gq == NGZ - 1;
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const int y = ty + r * ROWS;
@@ -595,8 +599,8 @@ __global__ __launch_bounds__(WG) void k_jacobi2(const J2Args a)
                     const T c = P1[r].v[v];
                     const T xm = v == 0 ? xl : P1[r].v[v - 1];
                     const T xp = v == VEC - 1 ? xr : P1[r].v[v + 1];
-                    const T zlo = (MIR && fzl != (T)0) ? c * fzl : P0[r].v[v];
-                    const T zhi = (MIR && fzh != (T)0) ? c * fzh : P2[r].v[v];
+                    const T zlo = MIR && ozl ? c * gzl.f : P0[r].v[v];
+                    const T zhi = MIR && ozh ? c * gzh.f : P2[r].v[v];
                     res.v[v] = upd(c, xm, xp, ym.v[v], yp.v[v], zlo, zhi, FQ[r].v[v], cm, cp, wd);
                 }
                 store_nt<T, VEC>(oq + x0 + NX * (y0 + y), res);
